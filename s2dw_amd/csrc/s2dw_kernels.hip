@@ -2742,54 +2742,52 @@ __device__ __forceinline__ void beta_syn_body(const BetaSynArgs &a, const double
   }
 }
 
-// Kernels over one scale (grid = the scale's workgroups).
-template <int LOGM, int BL>
-__global__ __launch_bounds__(kTN, 3) void k_beta_ana_t(const BetaAnaArgs a, int nmt) {
-  __shared__ double2 lds[lpad_size(kTS)];
-  beta_ana_body<LOGM, BL>(a, nmt, lds, blockIdx.x, gridDim.x);
-}
-template <int LOGM, int BL>
-__global__ __launch_bounds__(kTN, 3) void k_alpha_c2r_t(const AlphaArgs a, int npt) {
-  __shared__ double2 lds[lpad_size(kTS)];
-  alpha_c2r_body<LOGM, BL>(a, npt, lds, blockIdx.x, gridDim.x);
-}
-template <int LOGM, int BL>
-__global__ __launch_bounds__(kTN, 3) void k_alpha_r2c_t(const AlphaArgs a, int npt) {
-  __shared__ double2 lds[lpad_size(kTS)];
-  alpha_r2c_body<LOGM, BL>(a, npt, lds, blockIdx.x, gridDim.x);
-}
-template <int LOGM, int BL>
-__global__ __launch_bounds__(kTN, 3) void k_beta_syn_t(const BetaSynArgs a, int nmt) {
-  __shared__ double2 lds[lpad_size(kTS)];
-  beta_syn_body<LOGM, BL>(a, a.V, a.Vt, a.tw8, nmt, lds, blockIdx.x, gridDim.x);
-}
+// Kernels over one scale or over two scales of the same shape (the full-band
+// scales 0 and 1: only their data pointers differ): workgroups below `half`
+// run the first argument set, the others the second; one scale has half =
+// gridDim.x.  The workgroup holds nt_of(LOGM) threads with kTE slots each:
+// kTN threads up to M = kTS, and one sequence of M = 2^LOGM slots beyond
+// (512 threads for 4096: band limits 513..1024; 1024 threads for 8192: band
+// limits above 1024; their slots are dynamic LDS).
+__host__ __device__ constexpr int nt_of(int logm) { return logm > kLogTS ? (1 << logm) / kTE : kTN; }
+__host__ __device__ constexpr int lds_of(int logm) { return logm > kLogTS ? (1 << logm) * (int)sizeof(double2) : 0; }
+// waves per SIMD: three of the kTN-thread engine (168 VGPRs), four beyond
+// (two 512-thread workgroups or one of 1024 share a CU, 128 VGPRs)
+__host__ __device__ constexpr int occ_of(int logm) { return logm > kLogTS ? 4 : 3; }
+// largest work length, and the LDS the beta stage's column sums add to the slots
+constexpr int kBigLogM = 13, kCsumLds = nt_of(kBigLogM) * (int)sizeof(double2) + 64;
+inline bool big_fft(const FftSpec &f) { return f.bluestein && f.M > kTS && f.M <= 1 << kBigLogM; }
+#define S2DW_SLOTS(LOGM)                                            \
+  extern __shared__ double2 dyn_lds[];                              \
+  __shared__ double2 fix_lds[(LOGM) > kLogTS ? 1 : lpad_size(kTS)]; \
+  double2 *lds = (LOGM) > kLogTS ? dyn_lds : fix_lds;
 
-// Kernels over two scales of the same shape (the full-band scales 0 and 1):
-// the first half of the grid runs the first argument set, the second half
-// the second (only their data pointers differ).
 template <int LOGM, int BL>
-__global__ __launch_bounds__(kTN, 3) void k_beta_ana_t2(const BetaAnaArgs a0, const BetaAnaArgs a1, int nmt) {
+__global__ __launch_bounds__(kTN, 3) void k_beta_ana_t2(const BetaAnaArgs a0, const BetaAnaArgs a1, int nmt, int half) {
   __shared__ double2 lds[lpad_size(kTS)];
-  const int half = gridDim.x >> 1, second = blockIdx.x >= (unsigned)half;
+  const bool second = (int)blockIdx.x >= half;
   beta_ana_body<LOGM, BL>(second ? a1 : a0, nmt, lds, blockIdx.x - (second ? half : 0), half);
 }
 template <int LOGM, int BL>
-__global__ __launch_bounds__(kTN, 3) void k_alpha_c2r_t2(const AlphaArgs a0, const AlphaArgs a1, int npt) {
-  __shared__ double2 lds[lpad_size(kTS)];
-  const int half = gridDim.x >> 1, second = blockIdx.x >= (unsigned)half;
-  alpha_c2r_body<LOGM, BL>(second ? a1 : a0, npt, lds, blockIdx.x - (second ? half : 0), half);
+__global__ __launch_bounds__(nt_of(LOGM), occ_of(LOGM)) void k_alpha_c2r_t2(const AlphaArgs a0, const AlphaArgs a1,
+                                                                           int npt, int half) {
+  S2DW_SLOTS(LOGM)
+  const bool second = (int)blockIdx.x >= half;
+  alpha_c2r_body<LOGM, BL, false, nt_of(LOGM)>(second ? a1 : a0, npt, lds, blockIdx.x - (second ? half : 0), half);
 }
 template <int LOGM, int BL>
-__global__ __launch_bounds__(kTN, 3) void k_alpha_c2r_t2m(const AlphaArgs a0, const AlphaArgs a1, int npt) {
-  __shared__ double2 lds[lpad_size(kTS)];
-  const int half = gridDim.x >> 1, second = blockIdx.x >= (unsigned)half;
-  alpha_c2r_body<LOGM, BL, true>(second ? a1 : a0, npt, lds, blockIdx.x - (second ? half : 0), half);
+__global__ __launch_bounds__(nt_of(LOGM), occ_of(LOGM)) void k_alpha_c2r_t2m(const AlphaArgs a0, const AlphaArgs a1,
+                                                                            int npt, int half) {
+  S2DW_SLOTS(LOGM)
+  const bool second = (int)blockIdx.x >= half;
+  alpha_c2r_body<LOGM, BL, true, nt_of(LOGM)>(second ? a1 : a0, npt, lds, blockIdx.x - (second ? half : 0), half);
 }
 template <int LOGM, int BL>
-__global__ __launch_bounds__(kTN, 3) void k_alpha_r2c_t2(const AlphaArgs a0, const AlphaArgs a1, int npt) {
-  __shared__ double2 lds[lpad_size(kTS)];
-  const int half = gridDim.x >> 1, second = blockIdx.x >= (unsigned)half;
-  alpha_r2c_body<LOGM, BL>(second ? a1 : a0, npt, lds, blockIdx.x - (second ? half : 0), half);
+__global__ __launch_bounds__(nt_of(LOGM), occ_of(LOGM)) void k_alpha_r2c_t2(const AlphaArgs a0, const AlphaArgs a1,
+                                                                           int npt, int half) {
+  S2DW_SLOTS(LOGM)
+  const bool second = (int)blockIdx.x >= half;
+  alpha_r2c_body<LOGM, BL, nt_of(LOGM)>(second ? a1 : a0, npt, lds, blockIdx.x - (second ? half : 0), half);
 }
 
 // Alpha stages of the full-band pair on the odd-length engine, length
@@ -2886,9 +2884,9 @@ __global__ __launch_bounds__(NT, 3) void k_alpha_r2c_o2(const AlphaArgs a0, cons
 }
 template <int LOGM, int BL>
 __global__ __launch_bounds__(kTN, 3) void k_beta_syn_t2(const BetaSynArgs a, const double2 *V1, double2 *Vt1,
-                                                        const double2 *tw81, int nmt) {
+                                                        const double2 *tw81, int nmt, int half) {
   __shared__ double2 lds[lpad_size(kTS)];
-  const int half = gridDim.x >> 1, second = blockIdx.x >= (unsigned)half;
+  const bool second = (int)blockIdx.x >= half;
   beta_syn_body<LOGM, BL>(a, second ? V1 : a.V, second ? Vt1 : a.Vt, second ? tw81 : a.tw8, nmt, lds,
                           blockIdx.x - (second ? half : 0), half);
 }
@@ -3070,57 +3068,25 @@ __device__ __forceinline__ void beta_syn_h2_body(const BetaSynArgs &a, const dou
   }
 }
 
-// Work length of the in-place FFT kernels for band limits above 1024: the
-// alpha lengths 2hi - 1 and beta lengths 2hi of 2049..4096 run through
-// Bluestein on 8192 points, one sequence per workgroup of 1024 threads.
-constexpr int kBigLogM = 13, kBigM = 1 << kBigLogM;
-constexpr int kBigLds = lpad_size(kBigM) * (int)sizeof(double2);  // 128 KiB
-inline bool big_fft(const FftSpec &f) { return f.bluestein && f.M == kBigM; }
-
-// One column per workgroup of M / 8 threads, work length M = 2^LOGM beyond
-// the 2048 slots of the kTN-thread engine (band limits above 1024: Bluestein
-// on 8192 points, 128 KiB of LDS in place); dynamic LDS of M slots.
-template <int LOGM>
-__global__ __launch_bounds__((1 << LOGM) / kTE) void k_beta_ana_hb(const BetaAnaArgs a, int nmt) {
-  extern __shared__ double2 lds[];
-  beta_ana_h2_body<LOGM, (1 << LOGM) / kTE, true>(a, nmt, lds, blockIdx.x, gridDim.x);
-}
-template <int LOGM>
-__global__ __launch_bounds__((1 << LOGM) / kTE) void k_beta_syn_hb(const BetaSynArgs a, int nmt) {
-  extern __shared__ double2 lds[];
-  __shared__ double2 csum[(1 << LOGM) / kTE];
-  beta_syn_h2_body<LOGM, (1 << LOGM) / kTE, true>(a, a.V, a.Vt, a.tw8, nmt, lds, csum, blockIdx.x, gridDim.x);
-}
-// alpha of a band limit above 1024: one row pair per workgroup, Bluestein
-// on M = 2^LOGM points in place.
-template <int LOGM>
-__global__ __launch_bounds__((1 << LOGM) / kTE) void k_alpha_c2r_big(const AlphaArgs a, int npt) {
-  extern __shared__ double2 lds[];
-  alpha_c2r_body<LOGM, 1, false, (1 << LOGM) / kTE>(a, npt, lds, blockIdx.x, gridDim.x);
-}
-template <int LOGM>
-__global__ __launch_bounds__((1 << LOGM) / kTE) void k_alpha_r2c_big(const AlphaArgs a, int npt) {
-  extern __shared__ double2 lds[];
-  alpha_r2c_body<LOGM, 1, (1 << LOGM) / kTE>(a, npt, lds, blockIdx.x, gridDim.x);
+template <int LOGM, bool BL>
+__global__ __launch_bounds__(nt_of(LOGM), occ_of(LOGM)) void k_beta_ana_h2(const BetaAnaArgs a0, const BetaAnaArgs a1,
+                                                                          int nmt, int half) {
+  S2DW_SLOTS(LOGM)
+  const bool second = (int)blockIdx.x >= half;
+  beta_ana_h2_body<LOGM, nt_of(LOGM), BL>(second ? a1 : a0, nmt, lds, blockIdx.x - (second ? half : 0), half);
 }
 
-template <int LOGM>
-__global__ __launch_bounds__(kTN, 3) void k_beta_ana_h2(const BetaAnaArgs a0, const BetaAnaArgs a1, int nmt) {
-  __shared__ double2 lds[lpad_size(kTS)];
-  const int half = gridDim.x >> 1, second = blockIdx.x >= (unsigned)half;
-  beta_ana_h2_body<LOGM>(second ? a1 : a0, nmt, lds, blockIdx.x - (second ? half : 0), half);
+template <int LOGM, bool BL>
+__global__ __launch_bounds__(nt_of(LOGM), occ_of(LOGM)) void k_beta_syn_h2(const BetaSynArgs a, const double2 *V1,
+                                                                          double2 *Vt1, const double2 *tw81, int nmt,
+                                                                          int half) {
+  S2DW_SLOTS(LOGM)
+  __shared__ double2 csum[nt_of(LOGM)];
+  const bool second = (int)blockIdx.x >= half;
+  beta_syn_h2_body<LOGM, nt_of(LOGM), BL>(a, second ? V1 : a.V, second ? Vt1 : a.Vt, second ? tw81 : a.tw8, nmt, lds,
+                                          csum, blockIdx.x - (second ? half : 0), half);
 }
-
-template <int LOGM>
-__global__ __launch_bounds__(kTN, 3) void k_beta_syn_h2(const BetaSynArgs a, const double2 *V1, double2 *Vt1,
-                                                        const double2 *tw81, int nmt) {
-  __shared__ double2 lds[lpad_size(kTS)];
-  __shared__ double2 csum[kTN];
-  const int half = gridDim.x >> 1, second = blockIdx.x >= (unsigned)half;
-  beta_syn_h2_body<LOGM>(a, second ? V1 : a.V, second ? Vt1 : a.Vt, second ? tw81 : a.tw8, nmt, lds, csum,
-                         blockIdx.x - (second ? half : 0), half);
-}
-
+#undef S2DW_SLOTS
 
 // ---------------------------------------------------------------------------
 // Grouped launches: several scales of one stage in a single grid (the two
@@ -3148,29 +3114,35 @@ __device__ __forceinline__ int seg_of(const SegTab &t, int b) {
   case 2 * (LM) + (B):             \
     BODY<LM, B>(__VA_ARGS__);      \
     break;
-// one-FFT-per-column beta bodies: selector kSelH2 + log2(2hi)
+// one-FFT-per-column beta bodies: selector kSelH2 + 2 log2(M) + bluestein
 constexpr int kSelH2 = 100;
-#define S2DW_SEL_H2(BODY, LM, ...) \
-  case kSelH2 + (LM):              \
-    BODY<LM>(__VA_ARGS__);         \
+#define S2DW_SEL_H2(BODY, LM, B, ...)     \
+  case kSelH2 + 2 * (LM) + (B):           \
+    BODY<LM, kTN, (B) != 0>(__VA_ARGS__); \
     break;
+#define S2DW_SEL_H2_ALL(BODY, ...)      \
+  S2DW_SEL_H2(BODY, 4, 0, __VA_ARGS__)  \
+  S2DW_SEL_H2(BODY, 5, 0, __VA_ARGS__)  \
+  S2DW_SEL_H2(BODY, 6, 0, __VA_ARGS__)  \
+  S2DW_SEL_H2(BODY, 7, 0, __VA_ARGS__)  \
+  S2DW_SEL_H2(BODY, 8, 0, __VA_ARGS__)  \
+  S2DW_SEL_H2(BODY, 9, 0, __VA_ARGS__)  \
+  S2DW_SEL_H2(BODY, 10, 0, __VA_ARGS__) \
+  S2DW_SEL_H2(BODY, 4, 1, __VA_ARGS__)  \
+  S2DW_SEL_H2(BODY, 5, 1, __VA_ARGS__)  \
+  S2DW_SEL_H2(BODY, 6, 1, __VA_ARGS__)  \
+  S2DW_SEL_H2(BODY, 7, 1, __VA_ARGS__)  \
+  S2DW_SEL_H2(BODY, 8, 1, __VA_ARGS__)  \
+  S2DW_SEL_H2(BODY, 9, 1, __VA_ARGS__)  \
+  S2DW_SEL_H2(BODY, 10, 1, __VA_ARGS__) \
+  S2DW_SEL_H2(BODY, 11, 1, __VA_ARGS__)
 
 __global__ __launch_bounds__(kTN, 3) void k_beta_ana_g(const SegTab t, const BetaAnaArgs *__restrict__ args) {
   __shared__ double2 lds[lpad_size(kTS)];
   const int s = seg_of(t, blockIdx.x), bid = blockIdx.x - t.first[s], nb = t.first[s + 1] - t.first[s];
   const BetaAnaArgs a = args[s];
   switch (t.sel[s]) {
-    S2DW_SEL(beta_ana_body, 5, 0, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(beta_ana_body, 6, 0, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(beta_ana_body, 7, 0, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(beta_ana_body, 8, 0, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(beta_ana_body, 9, 0, a, t.par[s], lds, bid, nb)
-    S2DW_SEL_H2(beta_ana_h2_body, 4, a, t.par[s], lds, bid, nb)
-    S2DW_SEL_H2(beta_ana_h2_body, 5, a, t.par[s], lds, bid, nb)
-    S2DW_SEL_H2(beta_ana_h2_body, 6, a, t.par[s], lds, bid, nb)
-    S2DW_SEL_H2(beta_ana_h2_body, 7, a, t.par[s], lds, bid, nb)
-    S2DW_SEL_H2(beta_ana_h2_body, 8, a, t.par[s], lds, bid, nb)
-    S2DW_SEL_H2(beta_ana_h2_body, 9, a, t.par[s], lds, bid, nb)
+    S2DW_SEL_H2_ALL(beta_ana_h2_body, a, t.par[s], lds, bid, nb)
     default: beta_ana_body<0, -1>(a, t.par[s], lds, bid, nb); break;
   }
 }
@@ -3188,6 +3160,7 @@ __global__ __launch_bounds__(kTN, 3) void k_alpha_c2r_g(const SegTab t, const Al
     S2DW_SEL(alpha_c2r_body, 8, 1, a, t.par[s], lds, bid, nb)
     S2DW_SEL(alpha_c2r_body, 9, 1, a, t.par[s], lds, bid, nb)
     S2DW_SEL(alpha_c2r_body, 10, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_c2r_body, 11, 1, a, t.par[s], lds, bid, nb)
     default: alpha_c2r_body<0, -1>(a, t.par[s], lds, bid, nb); break;
   }
 }
@@ -3205,6 +3178,7 @@ __global__ __launch_bounds__(kTN, 3) void k_alpha_c2r_gm(const SegTab t, const A
     S2DW_SEL(alpha_c2r_body_m, 8, 1, a, t.par[s], lds, bid, nb)
     S2DW_SEL(alpha_c2r_body_m, 9, 1, a, t.par[s], lds, bid, nb)
     S2DW_SEL(alpha_c2r_body_m, 10, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_c2r_body_m, 11, 1, a, t.par[s], lds, bid, nb)
     default: alpha_c2r_body<0, -1, true>(a, t.par[s], lds, bid, nb); break;
   }
 }
@@ -3222,6 +3196,7 @@ __global__ __launch_bounds__(kTN, 3) void k_alpha_r2c_g(const SegTab t, const Al
     S2DW_SEL(alpha_r2c_body, 8, 1, a, t.par[s], lds, bid, nb)
     S2DW_SEL(alpha_r2c_body, 9, 1, a, t.par[s], lds, bid, nb)
     S2DW_SEL(alpha_r2c_body, 10, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_r2c_body, 11, 1, a, t.par[s], lds, bid, nb)
     default: alpha_r2c_body<0, -1>(a, t.par[s], lds, bid, nb); break;
   }
 }
@@ -3232,22 +3207,13 @@ __global__ __launch_bounds__(kTN, 3) void k_beta_syn_g(const SegTab t, const Bet
   const int s = seg_of(t, blockIdx.x), bid = blockIdx.x - t.first[s], nb = t.first[s + 1] - t.first[s];
   const BetaSynArgs &a = args[s];
   switch (t.sel[s]) {
-    S2DW_SEL_H2(beta_syn_h2_body, 4, a, a.V, a.Vt, a.tw8, t.par[s], lds, csum, bid, nb)
-    S2DW_SEL_H2(beta_syn_h2_body, 5, a, a.V, a.Vt, a.tw8, t.par[s], lds, csum, bid, nb)
-    S2DW_SEL_H2(beta_syn_h2_body, 6, a, a.V, a.Vt, a.tw8, t.par[s], lds, csum, bid, nb)
-    S2DW_SEL_H2(beta_syn_h2_body, 7, a, a.V, a.Vt, a.tw8, t.par[s], lds, csum, bid, nb)
-    S2DW_SEL_H2(beta_syn_h2_body, 8, a, a.V, a.Vt, a.tw8, t.par[s], lds, csum, bid, nb)
-    S2DW_SEL_H2(beta_syn_h2_body, 9, a, a.V, a.Vt, a.tw8, t.par[s], lds, csum, bid, nb)
-    S2DW_SEL(beta_syn_body, 5, 0, a, a.V, a.Vt, a.tw8, t.par[s], lds, bid, nb)
-    S2DW_SEL(beta_syn_body, 6, 0, a, a.V, a.Vt, a.tw8, t.par[s], lds, bid, nb)
-    S2DW_SEL(beta_syn_body, 7, 0, a, a.V, a.Vt, a.tw8, t.par[s], lds, bid, nb)
-    S2DW_SEL(beta_syn_body, 8, 0, a, a.V, a.Vt, a.tw8, t.par[s], lds, bid, nb)
-    S2DW_SEL(beta_syn_body, 9, 0, a, a.V, a.Vt, a.tw8, t.par[s], lds, bid, nb)
+    S2DW_SEL_H2_ALL(beta_syn_h2_body, a, a.V, a.Vt, a.tw8, t.par[s], lds, csum, bid, nb)
     default: beta_syn_body<0, -1>(a, a.V, a.Vt, a.tw8, t.par[s], lds, bid, nb); break;
   }
 }
 #undef S2DW_SEL
 #undef S2DW_SEL_H2
+#undef S2DW_SEL_H2_ALL
 
 // Static layout wav(0:J,0:2B-2,0:2B-1,0:N-1) (jj fastest) <-> packed scales.
 // A workgroup covers 256 consecutive (jj, aa) entries of one row (b, g) of
@@ -3490,52 +3456,6 @@ WaveShape wave_shape(const Plan *p, const FftSpec &f) {
 // Workgroup engine: power-of-two work length 2 <= M <= kTS (kTS/2 when the
 // kernel holds both parities of a column); returns log2 of the sequences per
 // workgroup, or -1.
-// Launch of a team kernel specialised on the work length (M = 2^LOGM,
-// 32 <= M <= kTS; compile-time M folds the engine's LDS addressing into
-// immediate offsets) and on Bluestein vs direct; other lengths run the
-// generic instantiation <0, -1>, which reads both from the FftSpec.
-#define S2DW_TEAM_DISPATCH(KERN, F, GRID, STREAM, ...)                                           \
-  do {                                                                                          \
-    const int lg_ = 31 - __builtin_clz((unsigned)(F).M);                                        \
-    const bool bl_ = (F).bluestein != 0;                                                        \
-    const dim3 g_(GRID), b_(kTN);                                                               \
-    switch (bl_ ? lg_ : lg_ + 16) {                                                             \
-      case 5: hipLaunchKernelGGL((KERN<5, 1>), g_, b_, 0, STREAM, __VA_ARGS__); break;         \
-      case 6: hipLaunchKernelGGL((KERN<6, 1>), g_, b_, 0, STREAM, __VA_ARGS__); break;         \
-      case 7: hipLaunchKernelGGL((KERN<7, 1>), g_, b_, 0, STREAM, __VA_ARGS__); break;         \
-      case 8: hipLaunchKernelGGL((KERN<8, 1>), g_, b_, 0, STREAM, __VA_ARGS__); break;         \
-      case 9: hipLaunchKernelGGL((KERN<9, 1>), g_, b_, 0, STREAM, __VA_ARGS__); break;         \
-      case 10: hipLaunchKernelGGL((KERN<10, 1>), g_, b_, 0, STREAM, __VA_ARGS__); break;       \
-      case 11: hipLaunchKernelGGL((KERN<11, 1>), g_, b_, 0, STREAM, __VA_ARGS__); break;       \
-      case 21: hipLaunchKernelGGL((KERN<5, 0>), g_, b_, 0, STREAM, __VA_ARGS__); break;        \
-      case 22: hipLaunchKernelGGL((KERN<6, 0>), g_, b_, 0, STREAM, __VA_ARGS__); break;        \
-      case 23: hipLaunchKernelGGL((KERN<7, 0>), g_, b_, 0, STREAM, __VA_ARGS__); break;        \
-      case 24: hipLaunchKernelGGL((KERN<8, 0>), g_, b_, 0, STREAM, __VA_ARGS__); break;        \
-      case 25: hipLaunchKernelGGL((KERN<9, 0>), g_, b_, 0, STREAM, __VA_ARGS__); break;        \
-      case 26: hipLaunchKernelGGL((KERN<10, 0>), g_, b_, 0, STREAM, __VA_ARGS__); break;       \
-      case 27: hipLaunchKernelGGL((KERN<11, 0>), g_, b_, 0, STREAM, __VA_ARGS__); break;       \
-      default: hipLaunchKernelGGL((KERN<0, -1>), g_, b_, 0, STREAM, __VA_ARGS__); break;       \
-    }                                                                                           \
-  } while (0)
-
-// Pair launches (scales 0 and 1): specialised for the work lengths of the
-// full-band scales of common band limits, generic otherwise.
-#define S2DW_PAIR_DISPATCH(KERN, F, GRID, STREAM, ...)                                          \
-  do {                                                                                          \
-    const int lg_ = 31 - __builtin_clz((unsigned)(F).M);                                        \
-    const bool bl_ = (F).bluestein != 0;                                                        \
-    const dim3 g_(GRID), b_(kTN);                                                               \
-    switch (bl_ ? lg_ : lg_ + 16) {                                                             \
-      case 9: hipLaunchKernelGGL((KERN<9, 1>), g_, b_, 0, STREAM, __VA_ARGS__); break;         \
-      case 10: hipLaunchKernelGGL((KERN<10, 1>), g_, b_, 0, STREAM, __VA_ARGS__); break;       \
-      case 11: hipLaunchKernelGGL((KERN<11, 1>), g_, b_, 0, STREAM, __VA_ARGS__); break;       \
-      case 25: hipLaunchKernelGGL((KERN<9, 0>), g_, b_, 0, STREAM, __VA_ARGS__); break;        \
-      case 26: hipLaunchKernelGGL((KERN<10, 0>), g_, b_, 0, STREAM, __VA_ARGS__); break;       \
-      case 27: hipLaunchKernelGGL((KERN<11, 0>), g_, b_, 0, STREAM, __VA_ARGS__); break;       \
-      default: hipLaunchKernelGGL((KERN<0, -1>), g_, b_, 0, STREAM, __VA_ARGS__); break;       \
-    }                                                                                           \
-  } while (0)
-
 int team_logTw(const Plan *p, const FftSpec &f, bool pairs) {
   if (p->fft_engine != 0) return -1;
   const int M = f.M;
@@ -3545,7 +3465,113 @@ int team_logTw(const Plan *p, const FftSpec &f, bool pairs) {
   return lg;
 }
 
+int log2_of(int M) { return 31 - __builtin_clz((unsigned)M); }
 
+// Launch shape of a transform stage on the workgroup engine: work length
+// 2^lg, sequences (columns or row pairs) per workgroup, and whether the
+// one-FFT-per-column beta bodies run it.  lg < 0: the stage is not on the
+// engine (another engine was asked for, or a smooth length above 2048 that
+// runs directly).
+struct TeamShape {
+  int lg = -1, bl = 0, per = 0;
+  bool h2 = false;
+};
+
+// beta: one FFT per column for every Bluestein length (M from 16 to 8192)
+// and every power of two 2hi from 16 to kTS; the two-FFT bodies keep 2hi =
+// 2, 4, 8 (fewer columns than the engine's minimum) and plans that ask for
+// them.  Measured per full-band pair, synthesis: L = 397 (M = 2048) 52 us
+// against 492 us for two FFTs per column on the wave engine, L = 899
+// (M = 4096) 370 us against 2983 us on the two-buffer generic kernel;
+// analysis L = 1024 (2048 points, direct) 488 us against 1434 us.  The alpha
+// stage on M = 4096 in place: L = 1024 853 us against 1932 us (generic).
+TeamShape beta_shape(const Plan *p, const FftSpec &f, int hi) {
+  TeamShape r;
+  if (p->fft_engine != 0 || f.M < 2 || (f.M & (f.M - 1))) return r;
+  const int lg = log2_of(f.M);
+  r.bl = f.bluestein ? 1 : 0;
+  if ((p->beta_one || lg > kLogTS) && lg >= 4 && (f.bluestein ? lg <= kBigLogM && lds_of(lg) + kCsumLds <= p->max_lds : lg <= kLogTS)) {
+    r.lg = lg;
+    r.per = std::max(1, kTS >> lg);
+    r.h2 = true;
+    return r;
+  }
+  const int tl = team_logTw(p, f, true);
+  if (tl >= 0) {
+    r.lg = lg;
+    r.per = 1 << (tl - 1);
+  }
+  return r;
+}
+
+TeamShape alpha_shape(const Plan *p, const FftSpec &f) {
+  TeamShape r;
+  if (p->fft_engine != 0 || f.M < 2 || (f.M & (f.M - 1))) return r;
+  const int lg = log2_of(f.M);
+  if (lg > kLogTS && !(f.bluestein && lg <= kBigLogM && lds_of(lg) <= p->max_lds)) return r;
+  r.lg = lg;
+  r.bl = f.bluestein ? 1 : 0;
+  r.per = std::max(1, kTS >> lg);
+  return r;
+}
+
+// Launches of one scale (second set equal to the first, half = all
+// workgroups) or of the full-band pair.  The kernels are specialised on the
+// work length (compile-time M folds the engine's LDS addressing into
+// immediate offsets) and on Bluestein vs direct; lengths below 32 (alpha)
+// run the generic instantiation <0, -1>, which reads both from the FftSpec.
+#define S2DW_ALPHA_CASE(KERN, LM)                                                                              \
+  case LM:                                                                                                     \
+    hipLaunchKernelGGL((KERN<LM, 1>), g, dim3(nt_of(LM)), lds_of(LM), st, a0, a1, npt, half);                  \
+    break;
+#define S2DW_ALPHA_LAUNCH(NAME, KERN)                                                                          \
+  void NAME(const TeamShape &t, const AlphaArgs &a0, const AlphaArgs &a1, int npt, int half, int blocks,       \
+            hipStream_t st) {                                                                                  \
+    const dim3 g(blocks);                                                                                      \
+    switch (t.bl ? t.lg : 0) {                                                                                 \
+      S2DW_ALPHA_CASE(KERN, 5) S2DW_ALPHA_CASE(KERN, 6) S2DW_ALPHA_CASE(KERN, 7) S2DW_ALPHA_CASE(KERN, 8)      \
+      S2DW_ALPHA_CASE(KERN, 9) S2DW_ALPHA_CASE(KERN, 10) S2DW_ALPHA_CASE(KERN, 11) S2DW_ALPHA_CASE(KERN, 12)   \
+      S2DW_ALPHA_CASE(KERN, 13)                                                                                \
+      default: hipLaunchKernelGGL((KERN<0, -1>), g, dim3(kTN), 0, st, a0, a1, npt, half); break;               \
+    }                                                                                                          \
+  }
+S2DW_ALPHA_LAUNCH(launch_alpha_c2r, k_alpha_c2r_t2)
+S2DW_ALPHA_LAUNCH(launch_alpha_c2r_mom, k_alpha_c2r_t2m)
+S2DW_ALPHA_LAUNCH(launch_alpha_r2c, k_alpha_r2c_t2)
+#undef S2DW_ALPHA_LAUNCH
+#undef S2DW_ALPHA_CASE
+
+#define S2DW_H2_CASES(X) \
+  X(4, 0) X(5, 0) X(6, 0) X(7, 0) X(8, 0) X(9, 0) X(10, 0) X(11, 0) X(4, 1) X(5, 1) X(6, 1) X(7, 1) X(8, 1) X(9, 1) \
+  X(10, 1) X(11, 1) X(12, 1) X(13, 1)
+void launch_beta_ana(const TeamShape &t, const BetaAnaArgs &b0, const BetaAnaArgs &b1, int nmt, int half, int blocks,
+                     hipStream_t st) {
+  const dim3 g(blocks);
+  switch (t.h2 ? 2 * t.lg + t.bl : 0) {
+#define S2DW_X(LM, B)                                                                                               \
+  case 2 * (LM) + (B):                                                                                              \
+    hipLaunchKernelGGL((k_beta_ana_h2<LM, (B) != 0>), g, dim3(nt_of(LM)), lds_of(LM), st, b0, b1, nmt, half);       \
+    break;
+    S2DW_H2_CASES(S2DW_X)
+#undef S2DW_X
+    default: hipLaunchKernelGGL((k_beta_ana_t2<0, -1>), g, dim3(kTN), 0, st, b0, b1, nmt, half); break;
+  }
+}
+void launch_beta_syn(const TeamShape &t, const BetaSynArgs &y0, const BetaSynArgs &y1, int nmt, int half, int blocks,
+                     hipStream_t st) {
+  const dim3 g(blocks);
+  switch (t.h2 ? 2 * t.lg + t.bl : 0) {
+#define S2DW_X(LM, B)                                                                                                 \
+  case 2 * (LM) + (B):                                                                                                \
+    hipLaunchKernelGGL((k_beta_syn_h2<LM, (B) != 0>), g, dim3(nt_of(LM)), lds_of(LM), st, y0, y1.V, y1.Vt, y1.tw8, nmt, \
+                       half);                                                                                         \
+    break;
+    S2DW_H2_CASES(S2DW_X)
+#undef S2DW_X
+    default: hipLaunchKernelGGL((k_beta_syn_t2<0, -1>), g, dim3(kTN), 0, st, y0, y1.V, y1.Vt, y1.tw8, nmt, half); break;
+  }
+}
+#undef S2DW_H2_CASES
 
 }  // namespace
 
@@ -4021,9 +4047,11 @@ int plan_build(Plan *p, int B, int N, int J, double alpha, const double *K, cons
         auto it = slot.find(n);
         if (it == slot.end()) {
           FftSpec f{};
-          // alpha lengths (odd): Bluestein on the workgroup engine up to M = kTS;
-          // beta lengths hold both parities of a column: up to M = kTS / 2
-          const int maxM = p->fft_engine == 0 ? (which == 0 ? kTS : kTS / 2) : 0;
+          // lengths that are no power of two: Bluestein on the workgroup engine
+          // up to M = 4096 (2hi <= 2048), also where the length is smooth
+          // (L = 300: the beta stage of 600 points takes 45 us per scale as
+          // mixed-radix stages of the generic kernel)
+          const int maxM = p->fft_engine == 0 && (which == 0 || p->beta_one) ? 2 * kTS : p->fft_engine == 0 ? kTS / 2 : 0;
           if (int e = make_fft(p, n, &f, maxM)) return e;
           slot[n] = (int)p->ffts.size();
           p->ffts.push_back(f);
@@ -4086,9 +4114,9 @@ int plan_build(Plan *p, int B, int N, int J, double alpha, const double *K, cons
     (void)hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, p->device);
     p->max_lds = maxlds;
     size_t need = 0;
-    const bool big_ok = maxlds >= kBigLds + (int)(kBigM / kTE * sizeof(double2));
     for (const FftSpec &f : p->ffts)
-      if (!wave_shape(p, f).ok && !(big_ok && big_fft(f))) need = std::max(need, fft_lds(f, 0));
+      if (!wave_shape(p, f).ok && !(big_fft(f) && p->fft_engine == 0 && maxlds >= lds_of(log2_of(f.M)) + kCsumLds))
+        need = std::max(need, fft_lds(f, 0));
     if (need > (size_t)maxlds) {
       set_error("FFT work length needs %zu bytes of LDS, the device allows %d", need, maxlds);
       return kErrSizeInvalid;
@@ -4101,11 +4129,14 @@ int plan_build(Plan *p, int B, int N, int J, double alpha, const double *K, cons
                            (const void *)k_beta_syn_w<16>, (const void *)k_beta_syn_w<32>};
       for (const void *fn : fns) S2DW_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, maxlds));
     }
-    if (big_ok) {
-      const void *big[] = {(const void *)k_beta_ana_hb<kBigLogM>, (const void *)k_beta_syn_hb<kBigLogM>,
-                           (const void *)k_alpha_c2r_big<kBigLogM>, (const void *)k_alpha_r2c_big<kBigLogM>};
-      for (const void *fn : big) S2DW_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kBigLds));
-    }
+    const void *big[] = {(const void *)k_beta_ana_h2<12, true>, (const void *)k_beta_ana_h2<13, true>,
+                         (const void *)k_beta_syn_h2<12, true>, (const void *)k_beta_syn_h2<13, true>,
+                         (const void *)k_alpha_c2r_t2<12, 1>, (const void *)k_alpha_c2r_t2<13, 1>,
+                         (const void *)k_alpha_c2r_t2m<12, 1>, (const void *)k_alpha_c2r_t2m<13, 1>,
+                         (const void *)k_alpha_r2c_t2<12, 1>, (const void *)k_alpha_r2c_t2<13, 1>};
+    for (int i = 0; i < 10; ++i)
+      if (lds_of(12 + (i & 1)) + kCsumLds <= maxlds)
+        S2DW_HIP_CHECK(hipFuncSetAttribute(big[i], hipFuncAttributeMaxDynamicSharedMemorySize, lds_of(12 + (i & 1))));
   }
   p->d_cov = d_cov;
   p->d_Phi2 = nullptr;
@@ -4259,25 +4290,11 @@ BetaSynArgs make_beta_syn(const Plan *p, int j) {
   return b;
 }
 
-// Body selector of a grouped launch: 2 log2(M) + bluestein when the grouped
-// kernel has that specialisation (log2 M in [5, maxlog], Bluestein flag bl),
-// else 0 (generic body).
-// log2(2hi) when the beta stage of a scale with this FFT can run as one
-// FFT per column in a grouped launch (direct power of two 16 <= 2hi <= 512),
-// else 0
-int h2_log(const Plan *p, const FftSpec &f, int hi) {
-  if (!p->beta_one || f.bluestein || f.M != 2 * hi || (f.M & (f.M - 1))) return 0;
-  int lg = 0;
-  while ((1 << lg) < f.M) ++lg;
-  return lg >= 4 && lg <= 9 ? lg : 0;
-}
-
-int group_sel(const FftSpec &f, int maxlog, int bl) {
-  int lg = 0;
-  while ((1 << lg) < f.M) ++lg;
-  const int b = f.bluestein ? 1 : 0;
-  return (lg >= 5 && lg <= maxlog && b == bl) ? 2 * lg + b : 0;
-}
+// Body selector of a grouped alpha launch: 2 log2(M) + bluestein for the
+// specialised work lengths (Bluestein, log2 M in [5, 11]), else 0 (generic).
+int alpha_sel(const TeamShape &t) { return t.bl && t.lg >= 5 && t.lg <= kLogTS ? 2 * t.lg + 1 : 0; }
+// ... of a grouped beta launch
+int beta_sel(const TeamShape &t) { return t.h2 ? kSelH2 + 2 * t.lg + t.bl : 0; }
 
 // Grouped launches (all on the workgroup FFT engine): the two full-band
 // scales j = 0, 1 (same shapes) in one launch per stage on the main stream,
@@ -4314,6 +4331,7 @@ int build_group(Plan *p, GroupState *gs, int gi, int j0, int j1) {
   std::vector<BetaAnaArgs> ba;
   std::vector<AlphaArgs> ac, ar;
   std::vector<BetaSynArgs> bs;
+  std::vector<int> taken;
   bool ok = j1 - j0 >= 2 || (gi == 1 && j1 > j0);
   const bool syn_ok = nn > 0 && N <= kMaxCol;
   for (int j = j0; j < j1 && ok; ++j) {
@@ -4325,32 +4343,26 @@ int build_group(Plan *p, GroupState *gs, int gi, int j0, int j1) {
     BetaAnaArgs b = make_beta_ana(p, j);
     AlphaArgs a = make_alpha(p, j, false), r = make_alpha(p, j, true);
     BetaSynArgs y = make_beta_syn(p, j);
-    const int tb = team_logTw(p, b.f, true), ta = team_logTw(p, a.f, false);
-    if (tb < 0 || ta < 0) {
-      ok = false;
-      break;
+    // scales beyond the kTN-thread engine's slots launch one by one
+    const TeamShape tb = beta_shape(p, b.f, s.hi), ta = alpha_shape(p, a.f);
+    if (tb.lg < 0 || ta.lg < 0 || tb.lg > kLogTS || ta.lg > kLogTS || (tb.h2 && !tb.bl && tb.lg == kLogTS)) {
+      ok = gi == 1 && j0 > 0;
+      continue;
     }
-    b.logT = y.logT = tb;
-    a.logT = r.logT = ta;
-    const int nmt = (s.hi + (1 << (tb - 1)) - 1) >> (tb - 1), npt = (s.hi + (1 << ta) - 1) >> ta;
+    b.logT = y.logT = team_logTw(p, b.f, true);
+    a.logT = r.logT = team_logTw(p, a.f, false);
+    const int nmt = (s.hi + tb.per - 1) / tb.per, npt = (s.hi + ta.per - 1) / ta.per;
     auto add = [](SegTab &t, int blocks, int sel, int par) {
       const int i = t.nseg++;
       t.first[i + 1] = t.first[i] + blocks;
       t.sel[i] = sel;
       t.par[i] = par;
     };
-    // beta: one FFT per column (kSelH2) for power-of-two 2hi from 16 to 512
-    const int lb = h2_log(p, b.f, s.hi);
-    if (lb > 0) {
-      const int nmh = (s.hi + (kTS >> lb) - 1) / (kTS >> lb);
-      add(G.ba, nmh * N, kSelH2 + lb, nmh);
-      add(G.bs, nmh * nn, kSelH2 + lb, nmh);
-    } else {
-      add(G.ba, nmt * N, group_sel(b.f, 10, 0), nmt);
-      add(G.bs, nmt * nn, group_sel(y.f, 10, 0), nmt);
-    }
-    add(G.ac, npt * N, group_sel(a.f, 11, 1), npt);
-    add(G.ar, npt * N, group_sel(r.f, 11, 1), npt);
+    add(G.ba, nmt * N, beta_sel(tb), nmt);
+    add(G.bs, nmt * nn, beta_sel(tb), nmt);
+    add(G.ac, npt * N, alpha_sel(ta), npt);
+    add(G.ar, npt * N, alpha_sel(ta), npt);
+    taken.push_back(j);
     const int gj = G.gm.nseg++;
     G.gm.first[gj + 1] = G.gm.first[gj] + (int)((2LL * s.hi * s.hi + 255) / 256);
     G.gm.g[gj] = GammaSeg{p->d_tb + s.tb_off, p->d_wq + p->wq_off[j], s.hi};
@@ -4364,11 +4376,10 @@ int build_group(Plan *p, GroupState *gs, int gi, int j0, int j1) {
   G.ana = ok;
   G.syn = ok && syn_ok;
   if (!ok) return kErrNone;
-  for (int j = j0; j < j1; ++j)
-    if (!scale_empty(p->sc[j])) {
-      gs->in_ana[j] = 1;
-      gs->in_syn[j] = G.syn;
-    }
+  for (int j : taken) {
+    gs->in_ana[j] = 1;
+    gs->in_syn[j] = G.syn;
+  }
   DevAlloc da{p};
   if (int e = da.alloc(&G.d_ba, ba.size())) return e;
   if (int e = da.alloc(&G.d_ac, ac.size())) return e;
@@ -4402,9 +4413,9 @@ int build_groups(Plan *p) {
     const Scale &s = p->sc[j];
     long long r = 0;
     if (!scale_empty(s)) {
-      const int ta = team_logTw(p, p->ffts[s.fa], false);
-      if (ta < 0) mok = false;
-      else r = (long long)((s.hi + (1 << ta) - 1) >> ta) * N;
+      const TeamShape ta = alpha_shape(p, p->ffts[s.fa]);
+      if (ta.lg < 0) mok = false;
+      else r = (long long)((s.hi + ta.per - 1) / ta.per) * N;
     }
     p->momf_rec0[j + 1] = p->momf_rec0[j] + r;
   }
@@ -4429,7 +4440,7 @@ int build_groups(Plan *p) {
   // FFT specs and run on the workgroup engine
   if (!all_in && Jp1 >= 2 && !scale_empty(p->sc[0]) && !scale_empty(p->sc[1]) && p->sc[0].fa == p->sc[1].fa &&
       p->sc[0].fb == p->sc[1].fb && p->sc[0].hi == p->sc[1].hi &&
-      team_logTw(p, p->ffts[p->sc[0].fb], true) >= 0 && team_logTw(p, p->ffts[p->sc[0].fa], false) >= 0)
+      beta_shape(p, p->ffts[p->sc[0].fb], p->sc[0].hi).lg >= 0 && alpha_shape(p, p->ffts[p->sc[0].fa]).lg >= 0)
     gs->pair = true;
   for (int j = 0; j < Jp1; ++j)
     if (!scale_empty(p->sc[j]) && !gs->in_ana[j] && !(gs->pair && j < 2)) mok = false;
@@ -4617,24 +4628,18 @@ int run_analysis(Plan *p, double *d_wav, double2 *d_scoeff, const double2 *d_flm
   const bool pair = grp && grp->pair;
   if (pair) {
     BetaAnaArgs b0 = make_beta_ana(p, 0), b1 = make_beta_ana(p, 1);
-    const int tb = team_logTw(p, b0.f, true);
-    b0.logT = b1.logT = tb;
-    const int nmt = (p->sc[0].hi + (1 << (tb - 1)) - 1) >> (tb - 1);
+    b0.logT = b1.logT = team_logTw(p, b0.f, true);
     if (!refb) {
       StageTimer tm(p, 2);
-      const int M = b0.f.M, nmh = (p->sc[0].hi + kTS / M - 1) / (kTS / M);
-      if (p->beta_one && !b0.f.bluestein && M == 1024)
-        hipLaunchKernelGGL(k_beta_ana_h2<10>, dim3(2 * nmh * N), dim3(kTN), 0, st, b0, b1, nmh);
-      else if (p->beta_one && !b0.f.bluestein && M == 512)
-        hipLaunchKernelGGL(k_beta_ana_h2<9>, dim3(2 * nmh * N), dim3(kTN), 0, st, b0, b1, nmh);
-      else
-        S2DW_PAIR_DISPATCH(k_beta_ana_t2, b0.f, 2 * nmt * N, st, b0, b1, nmt);
+      const TeamShape tb = beta_shape(p, b0.f, b0.hi);
+      const int nmt = (b0.hi + tb.per - 1) / tb.per;
+      launch_beta_ana(tb, b0, b1, nmt, nmt * N, 2 * nmt * N, st);
       S2DW_HIP_CHECK(hipGetLastError());
     }
     AlphaArgs a0 = make_alpha(p, 0, false), a1 = make_alpha(p, 1, false);
-    const int ta = team_logTw(p, a0.f, false);
-    a0.logT = a1.logT = ta;
-    const int npt = (p->sc[0].hi + (1 << ta) - 1) >> ta;
+    const TeamShape ta = alpha_shape(p, a0.f);
+    a0.logT = a1.logT = team_logTw(p, a0.f, false);
+    const int npt = (a0.hi + ta.per - 1) / ta.per;
     StageTimer tm(p, 3);
     if (d_mom) {
       a0.mp = p->d_momf + 8 * p->momf_rec0[0];
@@ -4646,7 +4651,7 @@ int run_analysis(Plan *p, double *d_wav, double2 *d_scoeff, const double2 *d_flm
         hipLaunchKernelGGL((k_alpha_c2r_o2<31, 11, 3, kOddNT, kOddT, kOddSplit, true>), dim3(2 * npo * N),
                            dim3(kOddNT), 0, st, a0, a1, npo, p->d_otw);
       else
-        S2DW_PAIR_DISPATCH(k_alpha_c2r_t2m, a0.f, 2 * npt * N, st, a0, a1, npt);
+        launch_alpha_c2r_mom(ta, a0, a1, npt, npt * N, 2 * npt * N, st);
     } else {
       a0.W = d_wav + p->sc[0].wav_off;
       a1.W = d_wav + p->sc[1].wav_off;
@@ -4654,7 +4659,7 @@ int run_analysis(Plan *p, double *d_wav, double2 *d_scoeff, const double2 *d_flm
         const int npo = (kOddHi + kOddT - 1) / kOddT;
         hipLaunchKernelGGL((k_alpha_c2r_o2<31, 11, 3>), dim3(2 * npo * N), dim3(kOddNT), 0, st, a0, a1, npo, p->d_otw);
       } else {
-        S2DW_PAIR_DISPATCH(k_alpha_c2r_t2, a0.f, 2 * npt * N, st, a0, a1, npt);
+        launch_alpha_c2r(ta, a0, a1, npt, npt * N, 2 * npt * N, st);
       }
     }
     S2DW_HIP_CHECK(hipGetLastError());
@@ -4683,19 +4688,17 @@ int run_analysis(Plan *p, double *d_wav, double2 *d_scoeff, const double2 *d_flm
       b.Tb = p->d_tb + s.tb_off;
       b.tw8 = p->d_tw8 + p->tw8_off[j];
       const WaveShape ws = wave_shape(p, b.f);
-      const int tl = team_logTw(p, b.f, true);
-      if (tl >= 0) {
-        b.logT = tl;
-        const int MC = 1 << (tl - 1), nmt = (s.hi + MC - 1) / MC;
-        S2DW_TEAM_DISPATCH(k_beta_ana_t, b.f, nmt * N, sj, b, nmt);
+      const TeamShape ts = beta_shape(p, b.f, s.hi);
+      if (ts.lg >= 0) {
+        b.logT = team_logTw(p, b.f, true);
+        const int nmt = (s.hi + ts.per - 1) / ts.per;
+        launch_beta_ana(ts, b, b, nmt, nmt * N, nmt * N, sj);
       } else if (ws.ok) {
         b.logT = ws.logTw;
         const int TMW = ws.WPB << ws.logTw;
         const dim3 grid((s.hi + TMW - 1) / TMW, N, 2), block(64 * ws.WPB);
         if (ws.E == 16) hipLaunchKernelGGL(k_beta_ana_w<16>, grid, block, ws.lds, sj, b);
         else hipLaunchKernelGGL(k_beta_ana_w<32>, grid, block, ws.lds, sj, b);
-      } else if (big_fft(b.f)) {
-        hipLaunchKernelGGL(k_beta_ana_hb<kBigLogM>, dim3(s.hi * N), dim3(kBigM / kTE), kBigLds, sj, b, s.hi);
       } else {
         const int T = 1 << b.logT;
         const size_t lds = fft_lds(b.f, b.logT);
@@ -4713,19 +4716,17 @@ int run_analysis(Plan *p, double *d_wav, double2 *d_scoeff, const double2 *d_flm
       al.Tb = p->d_tb + s.tb_off;
       al.W = wj;
       const WaveShape ws = wave_shape(p, al.f);
-      const int tl = team_logTw(p, al.f, false);
-      if (tl >= 0) {
-        al.logT = tl;
-        const int npt = (s.hi + (1 << tl) - 1) >> tl;
-        S2DW_TEAM_DISPATCH(k_alpha_c2r_t, al.f, npt * N, sj, al, npt);
+      const TeamShape ts = alpha_shape(p, al.f);
+      if (ts.lg >= 0) {
+        al.logT = team_logTw(p, al.f, false);
+        const int npt = (s.hi + ts.per - 1) / ts.per;
+        launch_alpha_c2r(ts, al, al, npt, npt * N, npt * N, sj);
       } else if (ws.ok) {
         al.logT = ws.logTw;
         const int per = ws.WPB << ws.logTw;
         const dim3 grid((s.hi + per - 1) / per, N), block(64 * ws.WPB);
         if (ws.E == 16) hipLaunchKernelGGL(k_alpha_c2r_w<16>, grid, block, ws.lds, sj, al);
         else hipLaunchKernelGGL(k_alpha_c2r_w<32>, grid, block, ws.lds, sj, al);
-      } else if (big_fft(al.f)) {
-        hipLaunchKernelGGL(k_alpha_c2r_big<kBigLogM>, dim3(s.hi * N), dim3(kBigM / kTE), kBigLds, sj, al, s.hi);
       } else {
         const int T = 1 << al.logT;
         const size_t lds = fft_lds(al.f, al.logT);
@@ -4792,18 +4793,18 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
   }
   if (pair) {
     AlphaArgs a0 = make_alpha(p, 0, true), a1 = make_alpha(p, 1, true);
-    const int ta = team_logTw(p, a0.f, false);
-    a0.logT = a1.logT = ta;
+    const TeamShape ta = alpha_shape(p, a0.f);
+    a0.logT = a1.logT = team_logTw(p, a0.f, false);
     a0.W = const_cast<double *>(d_wav + p->sc[0].wav_off);
     a1.W = const_cast<double *>(d_wav + p->sc[1].wav_off);
-    const int npt = (p->sc[0].hi + (1 << ta) - 1) >> ta;
+    const int npt = (a0.hi + ta.per - 1) / ta.per;
     {
       StageTimer tm(p, 5);
       if (p->d_otw) {
         const int npo = (kOddHi + kOddT - 1) / kOddT;
         hipLaunchKernelGGL((k_alpha_r2c_o2<31, 11, 3>), dim3(2 * npo * N), dim3(kOddNT), 0, st, a0, a1, npo, p->d_otw);
       } else {
-        S2DW_PAIR_DISPATCH(k_alpha_r2c_t2, a0.f, 2 * npt * N, st, a0, a1, npt);
+        launch_alpha_r2c(ta, a0, a1, npt, npt * N, 2 * npt * N, st);
       }
       S2DW_HIP_CHECK(hipGetLastError());
     }
@@ -4825,16 +4826,10 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
       S2DW_HIP_CHECK(hipGetLastError());
     }
     BetaSynArgs y0 = make_beta_syn(p, 0), y1 = make_beta_syn(p, 1);
-    const int tb = team_logTw(p, y0.f, true);
-    y0.logT = y1.logT = tb;
-    const int nmt = (p->sc[0].hi + (1 << (tb - 1)) - 1) >> (tb - 1);
-    const int M = y0.f.M, nmh = (p->sc[0].hi + kTS / M - 1) / (kTS / M);
-    if (p->beta_one && !y0.f.bluestein && M == 1024)
-      hipLaunchKernelGGL(k_beta_syn_h2<10>, dim3(2 * nmh * nn_all), dim3(kTN), 0, st, y0, y1.V, y1.Vt, y1.tw8, nmh);
-    else if (p->beta_one && !y0.f.bluestein && M == 512)
-      hipLaunchKernelGGL(k_beta_syn_h2<9>, dim3(2 * nmh * nn_all), dim3(kTN), 0, st, y0, y1.V, y1.Vt, y1.tw8, nmh);
-    else
-      S2DW_PAIR_DISPATCH(k_beta_syn_t2, y0.f, 2 * nmt * nn_all, st, y0, y1.V, y1.Vt, y1.tw8, nmt);
+    const TeamShape tb = beta_shape(p, y0.f, y0.hi);
+    y0.logT = y1.logT = team_logTw(p, y0.f, true);
+    const int nmt = (y0.hi + tb.per - 1) / tb.per;
+    launch_beta_syn(tb, y0, y1, nmt, nmt * nn_all, 2 * nmt * nn_all, st);
     S2DW_HIP_CHECK(hipGetLastError());
   }
   for (int j = 0; j < Jp1; ++j) {
@@ -4853,19 +4848,17 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
       al.V = p->d_tb + s.tb_off;
       al.scale = (4.0 * (M_PI * M_PI) / (double)N) / (2.0 * s.hi - 1.0);
       const WaveShape ws = wave_shape(p, al.f);
-      const int tl = team_logTw(p, al.f, false);
-      if (tl >= 0) {
-        al.logT = tl;
-        const int npt = (s.hi + (1 << tl) - 1) >> tl;
-        S2DW_TEAM_DISPATCH(k_alpha_r2c_t, al.f, npt * N, sj, al, npt);
+      const TeamShape ts = alpha_shape(p, al.f);
+      if (ts.lg >= 0) {
+        al.logT = team_logTw(p, al.f, false);
+        const int npt = (s.hi + ts.per - 1) / ts.per;
+        launch_alpha_r2c(ts, al, al, npt, npt * N, npt * N, sj);
       } else if (ws.ok) {
         al.logT = ws.logTw;
         const int per = ws.WPB << ws.logTw;
         const dim3 grid((s.hi + per - 1) / per, N), block(64 * ws.WPB);
         if (ws.E == 16) hipLaunchKernelGGL(k_alpha_r2c_w<16>, grid, block, ws.lds, sj, al);
         else hipLaunchKernelGGL(k_alpha_r2c_w<32>, grid, block, ws.lds, sj, al);
-      } else if (big_fft(al.f)) {
-        hipLaunchKernelGGL(k_alpha_r2c_big<kBigLogM>, dim3(s.hi * N), dim3(kBigM / kTE), kBigLds, sj, al, s.hi);
       } else {
         const int T = 1 << al.logT;
         const size_t lds = fft_lds(al.f, al.logT);
@@ -4899,9 +4892,8 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
           }
       }
       const WaveShape ws = wave_shape(p, b.f);
-      const int tl = team_logTw(p, b.f, true);
-      const bool big = !ws.ok && big_fft(b.f);
-      if (nn > 0 && (tl >= 0 || big) && N <= kMaxCol) {
+      const TeamShape ts = beta_shape(p, b.f, s.hi);
+      if (nn > 0 && ts.lg >= 0 && N <= kMaxCol) {
         const long long plane = 2LL * s.hi * s.hi;
         const dim3 gg((unsigned)((plane + 255) / 256));
         double2 *Vj = p->d_tb + s.tb_off;
@@ -4909,13 +4901,9 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
         else if (N <= 16) hipLaunchKernelGGL(k_gamma_syn<16>, gg, dim3(256), 0, sj, Vj, s.hi, N, nn, b.wq, b.eg);
         else hipLaunchKernelGGL(k_gamma_syn<32>, gg, dim3(256), 0, sj, Vj, s.hi, N, nn, b.wq, b.eg);
         S2DW_HIP_CHECK(hipGetLastError());
-        if (big) {
-          hipLaunchKernelGGL(k_beta_syn_hb<kBigLogM>, dim3(s.hi * nn), dim3(kBigM / kTE), kBigLds, sj, b, s.hi);
-        } else {
-          b.logT = tl;
-          const int MC = 1 << (tl - 1), nmt = (s.hi + MC - 1) / MC;
-          S2DW_TEAM_DISPATCH(k_beta_syn_t, b.f, nmt * nn, sj, b, nmt);
-        }
+        b.logT = team_logTw(p, b.f, true);
+        const int nmt = (s.hi + ts.per - 1) / ts.per;
+        launch_beta_syn(ts, b, b, nmt, nmt * nn, nmt * nn, sj);
         S2DW_HIP_CHECK(hipGetLastError());
       } else if (nn > 0 && ws.ok) {
         b.logT = ws.logTw;
