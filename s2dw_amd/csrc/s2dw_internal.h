@@ -84,6 +84,27 @@ struct Column {
   int part;  // 0: real part of S, 1: imaginary part
 };
 
+// Analysis contraction by parity of l (s2dw_anapar.hip): values of l per
+// group, m' (waves) per workgroup, and its arguments.
+constexpr int kParG = 8, kParWv = 4;
+struct AnaParArgs {
+  int L, N, rho;         // rho: 0 or 1, T_{-n} = (-1)^{m' + rho} (E - O)
+  const double2 *fT;     // [l][m], times i^{-m} (and i where S is imaginary)
+  const double *uinv;    // [l][m]
+  const double *rows;    // [rowA(m',l)]: A, Bc, columns n >= 0 of slot 0, of slot 1
+  long long rows_bytes;  // below 2^31
+  const double *S0;
+  const int *ends;       // per l, 8 ints: hi of the scale ending in slot 0 / 1 (0 none), low and high word of
+                         // its plane offset in Tg
+  const int *work;       // per workgroup: m'-block of kParWv | m-tile of 64 << 16
+  const int *gev;        // per aligned group of kParG l: bit k set when a scale ends at its l k
+  const int *gnext;      // per aligned group of kParG l: first l of the next group with an end (>= L: none)
+  const double *cg;      // gamma coefficients [2][NH + 1][2 NH]
+  double2 *Tg;
+};
+int par_rows(long long nrows, int NCa, int NH, int c0, const double *Ba, double *out, hipStream_t st);
+int par_contract(const AnaParArgs &a, int NH, hipStream_t st);
+
 // Optional per-stage HIP-event timing (stage ids in include/s2dw_hip.h).
 constexpr int kNumStages = 11;
 struct StageEvents {
@@ -180,6 +201,15 @@ struct Plan {
   int4 *d_swork = nullptr;    // MFMA synthesis work list
   int ana_p = 2;              // chains per lane in the VALU analysis contraction
   bool ana_mfma = true;       // analysis contraction on FP64 MFMA
+  int ana_nh = 0;             // columns n >= 0 of the contraction by parity of l (0: not available)
+  bool ana_par = false;       // ... and whether it runs
+  int ana_urot = 0;           // 1: S is imaginary
+  double *d_rows = nullptr;   // its rows
+  long long rows_bytes = 0;
+  int *d_ends = nullptr;      // its scale ends, and per group the end bits and the next group with an end
+  int *d_pgev = nullptr, *d_pgnext = nullptr;
+  int *d_awork = nullptr;     // its work list
+  double *d_cg = nullptr;     // its gamma coefficients
   bool ana_wave_indep = true; // ... with independent waves (else workgroup-staged operands)
   bool ana_mfma_ok = true, syn_mfma_ok = true;  // the MFMA contractions are available on this plan
   int fft_engine = 0;         // 0 workgroup engine, 1 wave engine, 2 generic Stockham

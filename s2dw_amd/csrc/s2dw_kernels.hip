@@ -27,37 +27,13 @@
 #include <map>
 #include <vector>
 
+#include "s2dw_dev.h"
 #include "s2dw_fft.h"
 #include "s2dw_internal.h"
 #include "s2dw_moments.h"
 
 namespace s2dw {
 
-constexpr int kMaxSc = 32;
-constexpr int kMaxCol = 32;
-constexpr int kChunk = 8;  // columns per contraction launch
-// Buffer descriptor word 3 for raw (untyped) loads on gfx9-family GPUs, and
-// an offset past the end of any buffer used with it: range-checked buffer
-// loads at that offset return 0, so a kernel can issue a load for every
-// lane unconditionally (buffers used this way stay below 2^31 bytes).
-constexpr int kBufWord3 = 0x00020000;
-constexpr unsigned kBufOut = 0x80000000u;
-constexpr long long kBufMaxBytes = 0x7fffffffLL;
-
-__host__ __device__ __forceinline__ long long tri0(long long l) { return l * (l + 1) / 2; }
-
-// Read-only tables indexed by wave-uniform values are read through the
-// constant address space so that the loads become scalar (s_load) and the
-// values feed v_fma_f64 as SGPR operands.
-typedef const double __attribute__((address_space(4))) *cdptr;
-__device__ __forceinline__ cdptr as_const(const double *p) { return (cdptr)(p); }
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-typedef const int __attribute__((address_space(4))) *ciptr;
-__device__ __forceinline__ ciptr as_const(const int *p) { return (ciptr)(p); }
-// analysis/thin row (m', l), m' <= l < L
-__host__ __device__ __forceinline__ long long rowA(long long mp, long long l, long long L) {
-  return mp * L - mp * (mp - 1) / 2 + (l - mp);
-}
 // synthesis row (l, m'), m' <= l
 __host__ __device__ __forceinline__ long long rowS(long long l, long long mp) { return tri0(l) + mp; }
 
@@ -95,15 +71,6 @@ __host__ __device__ __forceinline__ void mrec_coefs(int l, int mp, double *c1, d
   const double c = 1.0 / sqrt(a);
   *c1 = c;
   *c2 = sqrt((double)(l - mp) * (double)(l + mp + 1)) * c;
-}
-
-// start value of the l-chain of (m', m) at l0 = max(m', m)
-__device__ __forceinline__ double lchain_start(const double *__restrict__ S0, int mp, int m) {
-  if (mp >= m) {
-    const double v = S0[tri0(mp) + m];
-    return ((mp - m) & 1) ? -v : v;
-  }
-  return S0[tri0(m) + mp];
 }
 
 // ---------------------------------------------------------------------------
@@ -1810,9 +1777,10 @@ __global__ void k_flm_final_chunks(int L, int bl, int CW, const double2 *__restr
 // fT[l][m] = flm(l,m) for m <= l, 0 otherwise (32x32 tiles through LDS).
 // With sc: also the scaling coefficients (k_scoeff), from the first bl^2
 // threads of the grid (L^2 >= bl^2 of them): one launch fewer for plans that
-// run on one stream.
+// run on one stream.  rot >= 0: times i^{rot - m} (exact), which the
+// contraction by parity would apply to every output otherwise.
 __global__ void k_flm_to_fT(int L, const double2 *__restrict__ flm, double2 *__restrict__ fT, int bl,
-                            double2 *__restrict__ sc) {
+                            double2 *__restrict__ sc, int rot) {
   __shared__ double2 tile[32][33];
   const int l0 = blockIdx.x * 32, m0 = blockIdx.y * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 256 threads: 32 x 8
@@ -1827,7 +1795,11 @@ __global__ void k_flm_to_fT(int L, const double2 *__restrict__ flm, double2 *__r
   __syncthreads();
   for (int r = ty; r < 32; r += 8) {
     const int l = l0 + r, m = m0 + tx;
-    if (l < L && m < L) fT[(long long)l * L + m] = (m <= l) ? tile[tx][r] : make_double2(0.0, 0.0);
+    double2 x = (m <= l) ? tile[tx][r] : make_double2(0.0, 0.0);
+    const int k = rot < 0 ? 0 : (rot - m) & 3;
+    if (k & 1) x = make_double2(-x.y, x.x);
+    if (k & 2) x = make_double2(-x.x, -x.y);
+    if (l < L && m < L) fT[(long long)l * L + m] = x;
   }
 }
 
@@ -3854,6 +3826,88 @@ int plan_build(Plan *p, int B, int N, int J, double alpha, const double *K, cons
     hipLaunchKernelGGL(k_build_rows, dim3((unsigned)((nrows + 255) / 256)), dim3(256), 0, p->stream, ra);
     S2DW_HIP_CHECK(hipGetLastError());
   }
+  // contraction by parity of l (s2dw_anapar.hip): the streamed form with one
+  // real column per n (S all real or all imaginary, so that T_{-n} follows
+  // from T_n; an imaginary S(l,0) breaks the symmetry) and at most 4 columns
+  // n >= 0.  S2DW_HIP_ANA_KERNEL / S2DW_HIP_ANA_MFMA select another kernel.
+  if (!use_table && !split && NCa > 0) {
+    const int part = p->cols_a[0].part;
+    bool ok = NCa <= 8;
+    int nh = 0;
+    for (const Column &c : p->cols_a) {
+      ok = ok && c.part == part && !(c.n == 0 && part == 1);
+      nh += c.n >= 0;
+    }
+    ok = ok && nh <= 4 && N / 2 <= nh && 16LL * (L + 16) * L <= kBufMaxBytes &&
+         nrows * (2 + 2 * nh) * 8 + 4096 <= kBufMaxBytes;
+    if (ok) {
+      p->rows_bytes = nrows * (2 + 2 * nh) * (long long)sizeof(double);
+      p->ana_nh = nh;
+      p->ana_urot = part;
+      p->ana_par = !std::getenv("S2DW_HIP_ANA_KERNEL") && !std::getenv("S2DW_HIP_ANA_MFMA");
+      if (int e = da.alloc(&p->d_rows, (size_t)nrows * (2 + 2 * nh))) return e;
+      if (int e = par_rows(nrows, NCa, nh, NCa - nh, p->d_Ba, p->d_rows, p->stream)) return e;
+      // H(g, n) = i^n e^{i n pi g / N}: twice its real and imaginary part for
+      // n > 0 (the columns n and -n together), 1 and 0 for n = 0; the two
+      // orders put the real parts on the even-l or the odd-l sums
+      std::vector<double> cg((size_t)2 * (nh + 1) * 2 * nh, 0.0);
+      for (int g = 0; g <= nh; ++g)
+        for (int h = 0; h < nh; ++h) {
+          const int n = p->cols_a[NCa - nh + h].n;
+          const long double ang = pi * (long double)n * (0.5L + (long double)g / (long double)N);
+          const double cr = n == 0 ? 1.0 : (double)(2.0L * cosl(ang)), ci = n == 0 ? 0.0 : (double)(2.0L * sinl(ang));
+          double *c0 = cg.data() + (size_t)g * 2 * nh + h, *c1 = c0 + (size_t)(nh + 1) * 2 * nh;
+          c0[0] = c1[nh] = cr;
+          c0[nh] = c1[0] = ci;
+        }
+      if (int e = da.alloc(&p->d_cg, cg.size())) return e;
+      if (int e = upload(p->d_cg, cg.data(), cg.size() * sizeof(double), p->stream)) return e;
+      const int WV = kParWv, G = kParG, ngr = (L + G - 1) / G;
+      std::vector<int> ends((size_t)8 * L + 2 * (size_t)ngr, 0);
+      int *pev = ends.data() + 8 * (size_t)L, *pnx = pev + ngr;
+      for (int l = 0; l < L; ++l)
+        for (int sl = 0; sl < 2; ++sl) {
+          const int j = sl ? lflush[l].y : lflush[l].x;
+          if (j < 0) continue;
+          ends[8 * (size_t)l + sl] = p->sc[j].hi;
+          ends[8 * (size_t)l + 2 + 2 * sl] = (int)(unsigned)p->sc[j].tg_off;
+          ends[8 * (size_t)l + 3 + 2 * sl] = (int)(p->sc[j].tg_off >> 32);
+          pev[l / G] |= 1 << (l % G);
+        }
+      for (int q = ngr - 1; q >= 0; --q) pnx[q] = pev[q] ? G * q : q + 1 < ngr ? pnx[q + 1] : G * ngr;
+      // work list (WV m' x 64 m, L - max(m', m) values of l).  Workgroup i runs
+      // on XCD i % 8 and, while the grid is resident, on CU (i / 8) % 32 of
+      // it: every m-tile of an m'-block goes to one XCD, whose L2 then holds
+      // the block's rows; there longest first, every second run of 32
+      // reversed, so that a CU gets long and short ones
+      std::vector<int> cls[8], wk;
+      for (int y = 0; 64 * y < L; ++y)
+        for (int x = 0; WV * x < L; ++x) cls[x % 8].push_back(x | y << 16);
+      size_t pos[8] = {0};
+      for (auto &c : cls) {
+        std::stable_sort(c.begin(), c.end(), [WV](int u, int v) {
+          return std::max(WV * (u & 0xffff), 64 * (u >> 16)) < std::max(WV * (v & 0xffff), 64 * (v >> 16));
+        });
+        for (size_t i = 32; i < c.size(); i += 64)
+          std::reverse(c.begin() + (long)i, c.begin() + (long)std::min(i + 32, c.size()));
+      }
+      const size_t nwk = (size_t)((L + WV - 1) / WV) * ((L + 63) / 64);
+      for (size_t i = 0; wk.size() < nwk; ++i) {
+        int k = (int)(i % 8);
+        if (pos[k] >= cls[k].size())  // this class is used up: the fullest one
+          for (int q = 0; q < 8; ++q)
+            if (cls[q].size() - pos[q] > cls[k].size() - pos[k]) k = q;
+        wk.push_back(cls[k][pos[k]++]);
+      }
+      if (int e = da.alloc(&p->d_ends, ends.size())) return e;
+      p->d_pgev = p->d_ends + 8 * (size_t)L;
+      p->d_pgnext = p->d_pgev + ngr;
+      if (int e = upload(p->d_ends, ends.data(), ends.size() * sizeof(int), p->stream)) return e;
+      if (int e = da.alloc(&p->d_awork, wk.size())) return e;
+      if (int e = upload(p->d_awork, wk.data(), wk.size() * sizeof(int), p->stream)) return e;
+      S2DW_HIP_CHECK(hipStreamSynchronize(p->stream));  // the vectors are locals
+    }
+  }
   if (split) {
     if (int e = da.alloc(&p->d_Bq, (size_t)nrows * 16)) return e;
     p->bq_bytes = (long long)nrows * 16 * (long long)sizeof(uint4);
@@ -4529,7 +4583,7 @@ int run_analysis(Plan *p, double *d_wav, double2 *d_scoeff, const double2 *d_flm
   {
     StageTimer tm(p, 0);
     hipLaunchKernelGGL(k_flm_to_fT, dim3((L + 31) / 32, (L + 31) / 32), dim3(256), 0, st, L, d_flm, p->d_fT,
-                       p->bl_scoeff, sc_early ? d_scoeff : nullptr);
+                       p->bl_scoeff, sc_early ? d_scoeff : nullptr, p->ana_par ? p->ana_urot : -1);
     S2DW_HIP_CHECK(hipGetLastError());
   }
   // l-contraction, column chunks of kChunk
@@ -4554,7 +4608,26 @@ int run_analysis(Plan *p, double *d_wav, double2 *d_scoeff, const double2 *d_flm
     hipLaunchKernelGGL(k_fill, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (double *)p->d_tg, n);
     S2DW_HIP_CHECK(hipGetLastError());
   }
-  for (int c0 = 0; c0 < a.NCtot; c0 += kChunk) {
+  if (p->ana_par) {
+    StageTimer tm(p, 1);
+    AnaParArgs ap{};
+    ap.L = L;
+    ap.N = N;
+    ap.rho = (p->cols_a[0].n & 1) ^ p->ana_urot;
+    ap.fT = p->d_fT;
+    ap.uinv = p->d_uinv;
+    ap.rows = p->d_rows;
+    ap.S0 = p->d_S0;
+    ap.ends = p->d_ends;
+    ap.work = p->d_awork;
+    ap.gev = p->d_pgev;
+    ap.gnext = p->d_pgnext;
+    ap.rows_bytes = p->rows_bytes;
+    ap.cg = p->d_cg;
+    ap.Tg = p->d_tg;
+    if (int e = par_contract(ap, p->ana_nh, st)) return e;
+  }
+  for (int c0 = 0; c0 < (p->ana_par ? 0 : a.NCtot); c0 += kChunk) {
     StageTimer tm(p, 1);
     a.c0 = c0;
     a.accumulate = c0 > 0;
@@ -5117,6 +5190,7 @@ int plan_autotune(Plan *p, int reps, std::string *report) {
     const char *name;
     bool mfma, wave;
     int P;
+    bool par = false;
   };
   std::vector<AnaC> ac;
   // table form: the contraction kernels are fixed (only their table variants
@@ -5124,6 +5198,7 @@ int plan_autotune(Plan *p, int reps, std::string *report) {
   const bool fixed = p->d_Sa != nullptr, syn_fixed = p->tab_syn;
   if (fixed) *report += p->precision == 1 ? "analysis contraction: split (fixed);" : "analysis contraction: Wigner table form (fixed);";
   if (syn_fixed) *report += " synthesis contraction: Wigner table form (fixed);";
+  if (p->ana_nh > 0 && !fixed) ac.push_back({"parity", p->ana_mfma_ok, true, 2, true});
   if (p->ana_mfma_ok && !fixed) {
     ac.push_back({"mfma-wave", true, true, 2});
     ac.push_back({"mfma-staged", true, false, 2});
@@ -5135,6 +5210,7 @@ int plan_autotune(Plan *p, int reps, std::string *report) {
   size_t bi = 0;
   if (!fixed) *report += "analysis contraction:";
   for (size_t i = 0; i < ac.size(); ++i) {
+    p->ana_par = ac[i].par;
     p->ana_mfma = ac[i].mfma;
     p->ana_wave_indep = ac[i].wave;
     p->ana_p = ac[i].P;
@@ -5147,6 +5223,7 @@ int plan_autotune(Plan *p, int reps, std::string *report) {
     }
   }
   if (!fixed) {
+    p->ana_par = ac[bi].par;
     p->ana_mfma = ac[bi].mfma;
     p->ana_wave_indep = ac[bi].wave;
     p->ana_p = ac[bi].P;
