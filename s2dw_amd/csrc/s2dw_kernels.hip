@@ -1088,17 +1088,27 @@ __global__ void k_build_bq(long long nrows, int NCa, const double *__restrict__ 
 
 // Row exponents of the split kernel, per transform: e_m with
 // 2^{e_m} > max_{l} max(|Re f(l,m)|, |Im f(l,m)|) (0 for an all-zero row).
-__global__ void k_row_exp(int L, const double2 *__restrict__ fT, int *__restrict__ erow) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= L) return;
+// One workgroup per m over f_lm as the caller holds it, l fastest: the
+// reads are contiguous (L = 512: 3 us, against 145 us for one thread per m
+// walking down the columns of the transposed copy).
+__global__ __launch_bounds__(256) void k_row_exp(int L, const double2 *__restrict__ flm, int *__restrict__ erow) {
+  __shared__ double sh[4];
+  const int m = blockIdx.x;
   double mx = 0.0;
-  for (int l = m; l < L; ++l) {
-    const double2 v = fT[(long long)l * L + m];
+  for (int l = m + threadIdx.x; l < L; l += 256) {
+    const double2 v = flm[(long long)m * L + l];
     mx = fmax(mx, fmax(fabs(v.x), fabs(v.y)));
   }
-  int e = 0;
-  if (mx > 0.0) (void)frexp(mx, &e);  // mx < 2^e
-  erow[m] = e;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) mx = fmax(mx, __shfl_xor(mx, o));
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    mx = fmax(fmax(sh[0], sh[1]), fmax(sh[2], sh[3]));
+    int e = 0;
+    if (mx > 0.0) (void)frexp(mx, &e);  // mx < 2^e
+    erow[m] = e;
+  }
 }
 
 // u_m(l) = 1/sqrt((l+1)^2 - m^2) table [l][m] (0 where (l+1)^2 - m^2 <= 0).
@@ -4633,7 +4643,7 @@ int run_analysis(Plan *p, double *d_wav, double2 *d_scoeff, const double2 *d_flm
     a.accumulate = c0 > 0;
     const int nc = std::min(kChunk, a.NCtot - c0);
     if (p->precision == 1 && p->d_Bq) {
-      hipLaunchKernelGGL(k_row_exp, dim3((L + 255) / 256), dim3(256), 0, st, L, p->d_fT, p->d_erow);
+      hipLaunchKernelGGL(k_row_exp, dim3(L), dim3(256), 0, st, L, d_flm, p->d_erow);
       AnaSplitArgs as{a, p->d_gev, p->d_Sa, p->sa_doubles * 8, p->d_Bq, p->bq_bytes, p->d_erow};
       hipLaunchKernelGGL(k_ana_contract_split<kSplitD>, dim3((L + 3) / 4, (L + 15) / 16), dim3(256), 0, st, as);
       S2DW_HIP_CHECK(hipGetLastError());
