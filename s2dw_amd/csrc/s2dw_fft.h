@@ -761,6 +761,150 @@ __device__ __forceinline__ void team_fft_core(const FftSpec &s, double2 *buf, in
   }
 }
 
+// ---------------------------------------------------------------------------
+// Three-stage workgroup engine for a Bluestein convolution of M = 256 R3
+// points (R3 = 16: M = 4096 with 256 threads), 16 slots per thread, one
+// sequence per workgroup: radices 16, 16, R3 forward and R3, 16, 16 backward.
+// Three stages instead of the radix-8 engine's four, the first forward stage
+// from values the caller holds in registers, the last backward stage left in
+// registers, and the stages that meet at the filter joined in registers: the
+// slots are written four times and read four times per transform, where the
+// radix-8 engine of 512 threads writes and reads them eight times each and
+// spills (its four stages of twiddles stay in registers: 128 of 128 VGPRs;
+// here 2 waves per SIMD leave 256).
+// Physical slot of logical slot i: i ^ ((i >> 4) & 15); consecutive slots and
+// slots 16 apart, the two patterns of the stages, both fall in distinct
+// 16-byte bank groups over 16 lanes.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ int lpad16(int i) { return i ^ ((i >> 4) & 15); }
+
+// v[r] *= w^r (sign of DIR), r = 1..15, from w, w^2, w^4, w^8
+template <int DIR>
+__device__ __forceinline__ void twiddle16(double2 *v, double2 w1, double2 w2, double2 w4, double2 w8) {
+  double2 p[8];
+  p[1] = w1;
+  p[2] = w2;
+  p[3] = cmul(w1, w2);
+  p[4] = w4;
+  p[5] = cmul(w1, w4);
+  p[6] = cmul(w2, w4);
+  p[7] = cmul(p[3], w4);
+#pragma unroll
+  for (int r = 1; r < 8; ++r) v[r] = cmulw<DIR>(v[r], p[r]);
+  v[8] = cmulw<DIR>(v[8], w8);
+#pragma unroll
+  for (int r = 1; r < 8; ++r) v[8 + r] = cmulw<DIR>(v[8 + r], cmul(p[r], w8));
+}
+
+// 16-point DFT of v[0..7], v[8..15] = 0: the even outputs are the 8-point DFT
+// of v_r, the odd ones that of v_r w16^r.
+template <int DIR>
+__device__ __forceinline__ void dft16_half(double2 *v) {
+  constexpr double c1 = 0.92387953251128675613, s1 = 0.38268343236508977173, h = 0.70710678118654752440;
+  constexpr double cr[8] = {1.0, c1, h, s1, 0.0, -s1, -h, -c1}, ci[8] = {0.0, s1, h, c1, 1.0, c1, h, s1};
+  double2 a[8], b[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    a[r] = v[r];
+    b[r] = r == 0 ? v[0]
+         : r == 4 ? cmuli<DIR>(v[4])
+                  : make_double2(v[r].x * cr[r] - DIR * v[r].y * ci[r], v[r].y * cr[r] + DIR * v[r].x * ci[r]);
+  }
+  dft_small<8, DIR>(a);
+  dft_small<8, DIR>(b);
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    v[2 * q] = a[q];
+    v[2 * q + 1] = b[q];
+  }
+}
+
+// In: v[r], r < 8 = input k = threadIdx.x + NT r times chirp_k^{DIR} (zero for
+// k >= n; k >= M/2 is zero).  Out: v[r] = convolution output k = threadIdx.x
+// + NT r, to be multiplied by chirp_k^{DIR} (k < n <= M/2, so r < 8).  The
+// slots may be reused after a barrier.
+template <int LOGM, int DIR>
+__device__ __forceinline__ void team16_bluestein(const FftSpec &s, double2 *buf, double2 (&v)[16]) {
+  constexpr int M = 1 << LOGM, NT = M / 16, R3 = M / 256, NC = 16 / R3;
+  static_assert(R3 == 16 || R3 == 8, "M = 4096 or 2048");
+  const double2 *__restrict__ tw = s.tw;
+  const double2 *__restrict__ F = DIR > 0 ? s.filt_b : s.filt_f;
+  // forward, Ns = 1
+  dft16_half<-1>(v);
+  {
+    const int tid = stage_tid();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) buf[lpad16(16 * tid + r)] = v[r];
+  }
+  lds_barrier();
+  // forward, Ns = 16
+  {
+    const int tid = stage_tid(), jm = tid & 15, e = jm * (M / 256);
+    const double2 w1 = tw[e], w2 = tw[2 * e], w4 = tw[4 * e], w8 = tw[8 * e];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = buf[lpad16(tid + NT * r)];
+    lds_barrier();
+    twiddle16<-1>(v, w1, w2, w4, w8);
+    dft16<-1>(v);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) buf[lpad16((tid - jm) * 16 + jm + 16 * r)] = v[r];
+  }
+  lds_barrier();
+  // forward, Ns = 256 (radix R3), the filter, and backward, Ns = 1 (radix R3)
+  {
+    const int tid = stage_tid();
+    double2 f[16], w1[NC], w2[NC], w4[NC], w8[NC];
+#pragma unroll
+    for (int q = 0; q < NC; ++q) {
+      const int jj = tid + NT * q;
+      w1[q] = tw[jj];
+      w2[q] = tw[2 * jj];
+      w4[q] = tw[4 * jj];
+      w8[q] = R3 == 16 ? tw[8 * jj] : w4[q];
+#pragma unroll
+      for (int r = 0; r < R3; ++r) v[q * R3 + r] = buf[lpad16(jj + 256 * r)];
+#pragma unroll
+      for (int r = 0; r < R3; ++r) f[q * R3 + r] = F[jj + 256 * r];
+    }
+    lds_barrier();
+#pragma unroll
+    for (int q = 0; q < NC; ++q) {
+      double2 *x = v + q * R3;
+      if constexpr (R3 == 16) twiddle16<-1>(x, w1[q], w2[q], w4[q], w8[q]);
+      else twiddle_powers<R3, -1>(x, w1[q], w2[q], w4[q], w8[q]);
+      dft_pow2<R3, -1>(x);
+#pragma unroll
+      for (int r = 0; r < R3; ++r) x[r] = cmul(x[r], f[q * R3 + r]);
+      dft_pow2<R3, +1>(x);
+#pragma unroll
+      for (int r = 0; r < R3; ++r) buf[lpad16((tid + NT * q) * R3 + r)] = x[r];
+    }
+  }
+  lds_barrier();
+  // backward, Ns = R3
+  {
+    const int tid = stage_tid(), jm = tid & (R3 - 1), e = jm * 16;
+    const double2 w1 = tw[e], w2 = tw[2 * e], w4 = tw[4 * e], w8 = tw[8 * e];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = buf[lpad16(tid + NT * r)];
+    lds_barrier();
+    twiddle16<+1>(v, w1, w2, w4, w8);
+    dft16<+1>(v);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) buf[lpad16((tid - jm) * 16 + jm + R3 * r)] = v[r];
+  }
+  lds_barrier();
+  // backward, Ns = M/16
+  {
+    const int tid = stage_tid();
+    const double2 w1 = tw[tid], w2 = tw[2 * tid], w4 = tw[4 * tid], w8 = tw[8 * tid];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = buf[lpad16(tid + NT * r)];
+    twiddle16<+1>(v, w1, w2, w4, w8);
+    dft16<+1>(v);
+  }
+}
+
 // Workgroup id remapped so that consecutive logical tiles run on the same
 // XCD (the hardware deals workgroups to the 8 XCDs round-robin), which keeps
 // tiles that share cache lines in one L2.

@@ -1907,6 +1907,9 @@ struct AlphaArgs {
   double *W;          // per-scale wav [g][b][a]
   double2 *V;         // synthesis output
   double scale;       // synthesis scaling
+  const double2 *eg;  // synthesis: [ni][g] e^{-i n_ni pi g / N}
+  const double *wq;   // synthesis: 2hi quadrature weights
+  int N, nn, z0;      // synthesis: gamma samples, n-indices, the index of n = 0 (-1: none)
   long long woff;     // offset of W in the packed wavelet coefficients (grouped launches)
   double *mp;         // analysis reducing to moments: this scale's records (8 doubles per workgroup)
   long long moff;     // offset of mp in the plan's record buffer (grouped launches)
@@ -2597,7 +2600,185 @@ __device__ __forceinline__ void alpha_r2c_body(const AlphaArgs &a, int npt, doub
   }
 }
 
-// gamma-DFT and quadrature weights (synthesis), in place per (b, m):
+// ---------------------------------------------------------------------------
+// Synthesis alpha stage with the gamma-DFT and the quadrature weights in it.
+// The gamma-DFT commutes with the alpha transform, so it is taken first, on
+// the real wavelet rows while they are loaded:
+//   u_n(b, a) = sum_g w(g, b, a) e^{-i n pi g/N},
+//   U[ni][b][m] = scale wq[b] sum_a u_n(b, a) e^{-2 pi i m a/(2hi - 1)},  m < hi.
+// For n != 0 a row u_n(b, .) is complex and is one sequence whose outputs
+// m < hi are stored as they are; for n = 0 it is real and rows b, b + 1 are
+// packed into one sequence, unpacked by Hermitian symmetry.  With the n of
+// one parity that is N sequences per row pair, as many as the packed real rows
+// took, without the N planes V(g, b, m) being written and read again by a
+// gamma pass (L = 512, N = 8: 400 MB of 740 MB for the full-band pair); the
+// rows of a pair are read once per n-index, the repeats from L2 (the sequences
+// of a row pair are consecutive and so run on one XCD).
+// Sequence id q = (row pair) nseq + s, nseq = 2 nn - (z0 >= 0).
+// ---------------------------------------------------------------------------
+struct SynSeq {
+  int ni, b;    // n-index and row (the first row of the pair if packed)
+  bool packed;  // n = 0: rows b and b + 1
+};
+__device__ __forceinline__ int syn_nseq(const AlphaArgs &a) { return 2 * a.nn - (a.z0 >= 0 ? 1 : 0); }
+__device__ __forceinline__ SynSeq syn_seq(const AlphaArgs &a, int q) {
+  const int nseq = syn_nseq(a), p = (int)((unsigned)q / (unsigned)nseq);
+  int s = q - p * nseq;
+  if (a.z0 >= 0) {
+    if (s == 0) return {a.z0, 2 * p, true};
+    --s;
+  }
+  int ni = s >> 1;
+  if (a.z0 >= 0 && ni >= a.z0) ++ni;
+  return {ni, 2 * p + (s & 1), false};
+}
+
+// G consecutive gamma samples g0.. of the E samples at offsets o: every load
+// is issued before the first use.
+template <int E, int G>
+__device__ __forceinline__ void syn_gather_g(const double *__restrict__ W, const int (&o)[E], int gs, int g0, bool packed,
+                                             int n, const double2 *__restrict__ eg, double2 (&z)[E]) {
+  double w[G][E], w1[G][E];
+  double2 c[G];
+#pragma unroll
+  for (int i = 0; i < G; ++i) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) w[i][e] = W[o[e] + (g0 + i) * gs];
+    if (packed) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) w1[i][e] = W[o[e] + n + (g0 + i) * gs];
+    } else {
+      c[i] = eg[g0 + i];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < G; ++i)
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      if (packed) {
+        z[e].x += w[i][e];
+        z[e].y += w1[i][e];
+      } else {
+        z[e].x += w[i][e] * c[i].x;
+        z[e].y += w[i][e] * c[i].y;
+      }
+    }
+}
+
+// z[e] = u(sequence sq, sample k[e]), 0 for k[e] >= n or !on.  Up to four
+// gamma samples (4 E loads) in flight: with one at a time the loads' latency
+// was a third of the stage.
+template <int E>
+__device__ __forceinline__ void syn_gather(const AlphaArgs &a, const SynSeq &sq, bool on, const int (&k)[E],
+                                           double2 (&z)[E]) {
+  const int n = 2 * a.hi - 1, gs = 2 * a.hi * n, N = a.N;  // N gs <= 32 4096 4095 < 2^31
+  int o[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    z[e] = make_double2(0.0, 0.0);
+    o[e] = sq.b * n + (k[e] < n ? k[e] : 0);
+  }
+  const double2 *eg = a.eg + sq.ni * N;
+  if (sq.packed) {
+    int g = 0;
+    for (; g + 2 <= N; g += 2) syn_gather_g<E, 2>(a.W, o, gs, g, true, n, eg, z);
+    if (g < N) syn_gather_g<E, 1>(a.W, o, gs, g, true, n, eg, z);
+  } else {
+    int g = 0;
+    for (; g + 4 <= N; g += 4) syn_gather_g<E, 4>(a.W, o, gs, g, false, n, eg, z);
+    if (g + 2 <= N) {
+      syn_gather_g<E, 2>(a.W, o, gs, g, false, n, eg, z);
+      g += 2;
+    }
+    if (g < N) syn_gather_g<E, 1>(a.W, o, gs, g, false, n, eg, z);
+  }
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (!on || k[e] >= n) z[e] = make_double2(0.0, 0.0);
+}
+
+// stores output kk of a sequence (zp = Z(kk), zm = Z(n - kk), used for a
+// packed sequence only)
+__device__ __forceinline__ void syn_store(const AlphaArgs &a, const SynSeq &sq, int kk, double2 zp, double2 zm) {
+  double2 *u = a.V + ((long long)sq.ni * 2 * a.hi + sq.b) * a.hi;
+  if (sq.packed) {
+    const double h0 = 0.5 * a.scale * a.wq[sq.b], h1 = 0.5 * a.scale * a.wq[sq.b + 1];
+    u[kk] = make_double2(h0 * (zp.x + zm.x), h0 * (zp.y - zm.y));
+    u[a.hi + kk] = make_double2(h1 * (zp.y + zm.y), -h1 * (zp.x - zm.x));
+  } else {
+    const double h = a.scale * a.wq[sq.b];
+    u[kk] = make_double2(h * zp.x, h * zp.y);
+  }
+}
+
+// A thread works on one sequence: M/8 consecutive threads per sequence.  The
+// length 2hi - 1 is odd, so this is always Bluestein, n <= M/2, M >= 8.
+template <int LOGM, int, int NT = kTN>
+__device__ __forceinline__ void alpha_syn_body(const AlphaArgs &a, int, double2 *lds, int bid, int nb) {
+  constexpr int LOGTS = clog2(NT * kTE);
+  const FftSpec &f = a.f;
+  const int hi = a.hi, n = 2 * hi - 1, logM = LOGM > 0 ? LOGM : ilog2(f.M), M = 1 << logM;
+  const int logTw = LOGM > 0 ? LOGTS - LOGM : a.logT;
+  const int Q = hi * syn_nseq(a);
+  const int t0 = threadIdx.x >> (logM - 3), j0 = threadIdx.x & ((M >> 3) - 1);
+  const int tile0 = xcd_tile(bid, nb) << logTw;
+  const int q0 = tile0 + t0;
+  const bool on = q0 < Q;
+  SynSeq sq = syn_seq(a, on ? q0 : 0);
+  if constexpr (LOGM >= 9) {  // whole waves per sequence
+    sq.ni = uniform(sq.ni);
+    sq.b = uniform(sq.b);
+    sq.packed = uniform((int)sq.packed) != 0;
+  }
+  // samples k < M/2 only: slots k >= n are zero
+  int k[kTE / 2];
+  double2 z[kTE / 2];
+  if constexpr (LOGM > 0 && LOGM % 3 == 2) {
+    // the radix-4 first stage from the gathered rows: butterfly jj (slots
+    // jj + r M/4) has non-zero inputs for r < 2 only; the thread has
+    // butterflies j0 + i M/8, i < 2
+#pragma unroll
+    for (int i = 0; i < 4; ++i) k[i] = j0 + (M >> 3) * (i >> 1) + (M >> 2) * (i & 1);
+    syn_gather<4>(a, sq, on, k, z);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      double2 v[4];
+      v[0] = cmulw<-1>(z[2 * i], f.chirp[k[2 * i]]);  // the chirp table is zero for n <= k < M
+      v[1] = cmulw<-1>(z[2 * i + 1], f.chirp[k[2 * i + 1]]);
+      v[2] = v[3] = make_double2(0.0, 0.0);
+      dft_pow2<4, -1>(v);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) lds[lpad(((4 * k[2 * i] + r) << logTw) + t0)] = v[r];
+    }
+    lds_barrier();
+    team_fft_core<kTE, NT, -1, true>(f, lds, M, logTw, true, f.chirp_c);
+  } else {
+#pragma unroll
+    for (int e = 0; e < kTE / 2; ++e) k[e] = j0 + (M >> 3) * e;
+    syn_gather<kTE / 2>(a, sq, on, k, z);
+#pragma unroll
+    for (int e = 0; e < kTE / 2; ++e) {
+      lds[lpad((k[e] << logTw) + t0)] = cmulw<-1>(z[e], f.chirp[k[e]]);
+      lds[lpad(((k[e] + (M >> 1)) << logTw) + t0)] = make_double2(0.0, 0.0);
+    }
+    lds_barrier();
+    team_fft_core<kTE, NT, -1>(f, lds, M, logTw, true, f.chirp_c);
+  }
+  // outputs k < hi <= M/2
+  if (on)
+#pragma unroll
+    for (int e = 0; e < kTE / 2; ++e) {
+      const int kk = j0 + (M >> 3) * e;
+      if (kk < hi) {
+        const double2 zp = lds[lpad((kk << logTw) + t0)];
+        const double2 zm = sq.packed ? lds[lpad(((kk ? n - kk : 0) << logTw) + t0)] : zp;
+        syn_store(a, sq, kk, zp, zm);
+      }
+    }
+}
+
+// gamma-DFT and quadrature weights (synthesis) as a pass of its own, for the
+// stages whose alpha or beta kernels are not on the workgroup engine; in place per (b, m):
 // U[ni][b][m] = wq[b] sum_g V[g][b][m] e^{-i n_ni pi g/N}; ni < nn <= N <= NMAX.
 template <int NMAX>
 __device__ __forceinline__ void gamma_syn_body(double2 *V, int hi, int N, int nn, const double *__restrict__ wq,
@@ -2629,27 +2810,6 @@ template <int NMAX>
 __global__ __launch_bounds__(256) void k_gamma_syn(double2 *V, int hi, int N, int nn, const double *__restrict__ wq,
                                                    const double2 *__restrict__ eg) {
   gamma_syn_body<NMAX>(V, hi, N, nn, wq, eg, (long long)blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-// gamma-DFT of the small scales in one grid: segment s (scale) owns
-// workgroups [first[s], first[s+1]) and its plane V, weights wq and hi.
-struct GammaSeg {
-  double2 *V;
-  const double *wq;
-  int hi;
-};
-struct GammaTab {
-  int nseg;
-  int first[kMaxSc + 1];
-  GammaSeg g[kMaxSc];
-};
-
-template <int NMAX>
-__global__ __launch_bounds__(256) void k_gamma_syn_g(const GammaTab t, int N, int nn, const double2 *__restrict__ eg) {
-  int s = 0;
-  for (int i = 1; i < t.nseg; ++i) s = (int)blockIdx.x >= t.first[i] ? i : s;
-  const GammaSeg &g = t.g[s];
-  gamma_syn_body<NMAX>(g.V, g.hi, N, nn, g.wq, eg, (long long)(blockIdx.x - t.first[s]) * blockDim.x + threadIdx.x);
 }
 
 // beta (synthesis) for one n-index: sequence t = 2*mc + r holds column
@@ -2772,6 +2932,14 @@ __global__ __launch_bounds__(nt_of(LOGM), occ_of(LOGM)) void k_alpha_r2c_t2(cons
   alpha_r2c_body<LOGM, BL, nt_of(LOGM)>(second ? a1 : a0, npt, lds, blockIdx.x - (second ? half : 0), half);
 }
 
+template <int LOGM, int BL>
+__global__ __launch_bounds__(nt_of(LOGM), occ_of(LOGM)) void k_alpha_syn_t2(const AlphaArgs a0, const AlphaArgs a1,
+                                                                           int npt, int half) {
+  S2DW_SLOTS(LOGM)
+  const bool second = (int)blockIdx.x >= half;
+  alpha_syn_body<LOGM, BL, nt_of(LOGM)>(second ? a1 : a0, npt, lds, blockIdx.x - (second ? half : 0), half);
+}
+
 // Alpha stages of the full-band pair on the odd-length engine, length
 // n = 2hi - 1 = R0 R1 R2 (no Bluestein).  A workgroup holds kOddT row pairs
 // (each one packed complex sequence, as in alpha_c2r_body / alpha_r2c_body)
@@ -2831,39 +2999,130 @@ __global__ __launch_bounds__(NT, 3) void k_alpha_c2r_o2(const AlphaArgs a0, cons
   }
 }
 
-template <int R0, int R1, int R2, int NT = kOddNT, int T = kOddT, int SPLIT = kOddSplit>
-__global__ __launch_bounds__(NT, 3) void k_alpha_r2c_o2(const AlphaArgs a0, const AlphaArgs a1, int npt,
+// One sequence per workgroup (alpha_syn_body's ids and outputs).
+template <int R0, int R1, int R2, int NT = kOddNT, int SPLIT = kOddSplit>
+__global__ __launch_bounds__(NT, 3) void k_alpha_syn_o2(const AlphaArgs a0, const AlphaArgs a1,
                                                      const double2 *__restrict__ otw) {
-  constexpr int n = R0 * R1 * R2, hi = (n + 1) / 2;
-  __shared__ double2 lds[n * T];
+  constexpr int n = R0 * R1 * R2, hi = (n + 1) / 2, E = (n + NT - 1) / NT;
+  __shared__ double2 lds[n];
   const int half = gridDim.x >> 1, second = blockIdx.x >= (unsigned)half;
   const AlphaArgs &a = second ? a1 : a0;
-  const int tile = xcd_tile(blockIdx.x - (second ? half : 0), half);
-  const int g = tile / npt, p0 = (tile - g * npt) * T;
-  for (int idx = threadIdx.x; idx < n * T; idx += NT) {
-    const int t = idx % T, k = idx / T, pidx = p0 + t;
-    double2 z = make_double2(0.0, 0.0);
-    if (pidx < hi) {
-      const double *w0 = a.W + ((long long)g * 2 * hi + 2 * pidx) * n;
-      z = make_double2(w0[k], w0[n + k]);
-    }
-    lds[k * T + t] = z;
+  const SynSeq us = syn_seq(a, xcd_tile(blockIdx.x - (second ? half : 0), half));
+  {
+    int k[E];
+    double2 z[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) k[e] = threadIdx.x + NT * e;
+    syn_gather<E>(a, us, true, k, z);
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      if (k[e] < n) lds[k[e]] = z[e];
   }
   lds_barrier();
-  odd_fft<R0, R1, R2, -1, NT, T, SPLIT>(lds, otw);
-  // unpack the two rows' Hermitian halves, scaled (alpha_r2c_body)
-  const double h = 0.5 * a.scale;
-  for (int idx = threadIdx.x; idx < hi * T; idx += NT) {
-    const int t = idx % T, kk = idx / T, pidx = p0 + t;
-    if (pidx < hi) {
-      const double2 zp = lds[kk * T + t];
-      const double2 zm = lds[(kk ? n - kk : 0) * T + t];
-      double2 *v0 = a.V + ((long long)g * 2 * hi + 2 * pidx) * hi;
-      v0[kk] = make_double2(h * (zp.x + zm.x), h * (zp.y - zm.y));
-      v0[hi + kk] = make_double2(h * (zp.y + zm.y), -h * (zp.x - zm.x));
+  odd_fft<R0, R1, R2, -1, NT, 1, SPLIT>(lds, otw);
+  for (int kk = threadIdx.x; kk < hi; kk += NT) {
+    const double2 zp = lds[kk];
+    const double2 zm = us.packed ? lds[kk ? n - kk : 0] : zp;
+    syn_store(a, us, kk, zp, zm);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Alpha stages and one-FFT-per-column beta stages on the three-stage engine
+// (Bluestein, M = 2^LOGM, M/16 threads, one sequence or column per
+// workgroup): inputs go straight into the first stage's registers and outputs
+// leave from the last stage's; the slots carry only what another thread needs
+// (the mirrored halves of the packed rows and of the beta columns).
+// ---------------------------------------------------------------------------
+template <int LOGM, bool MOM>
+__global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_alpha_c2r16(const AlphaArgs a0, const AlphaArgs a1, int npt,
+                                                                    int half) {
+  constexpr int NT = (1 << LOGM) / 16;
+  extern __shared__ double2 dyn_lds[];
+  const bool second = (int)blockIdx.x >= half;
+  const AlphaArgs &a = second ? a1 : a0;
+  const int hi = a.hi, n = 2 * hi - 1, tile = xcd_tile(blockIdx.x - (second ? half : 0), half);
+  const int g = tile / npt, pidx = tile - g * npt;  // npt = hi
+  double2 v[16];
+  {
+    const double2 *rb = a.Tb + ((long long)g * 2 * hi + 2 * pidx) * hi;
+    double2 p[8], q[8], c[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int k = threadIdx.x + NT * r, kk = k < hi ? k : k < n ? n - k : 0;
+      p[r] = rb[kk];
+      q[r] = rb[hi + kk];
+      c[r] = a.f.chirp[k];  // zero for n <= k < M
+    }
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int k = threadIdx.x + NT * r;
+      const double2 z = k == 0  ? make_double2(p[r].x, q[r].x)
+                        : k < hi ? make_double2(p[r].x - q[r].y, p[r].y + q[r].x)
+                                 : make_double2(p[r].x + q[r].y, -p[r].y + q[r].x);
+      v[r] = k < n ? cmulw<+1>(z, c[r]) : make_double2(0.0, 0.0);
+    }
+  }
+  team16_bluestein<LOGM, +1>(a.f, dyn_lds, v);
+  if constexpr (MOM) {
+    double x[16], wt[16];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int k = threadIdx.x + NT * r;
+      const double2 z = cmulw<+1>(v[r], a.f.chirp[k]);
+      x[2 * r] = z.x;
+      x[2 * r + 1] = z.y;
+      wt[2 * r] = wt[2 * r + 1] = k < n ? 1.0 : 0.0;
+    }
+    mom_record<16, NT>(x, wt, 0.0, a.mp + 8LL * tile);
+    return;
+  }
+  double *w0 = a.W + ((long long)g * 2 * hi + 2 * pidx) * n;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const int k = threadIdx.x + NT * r;
+    if (k < n) {
+      const double2 z = cmulw<+1>(v[r], a.f.chirp[k]);
+      w0[k] = z.x;
+      w0[n + k] = z.y;
     }
   }
 }
+
+template <int LOGM>
+__global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_alpha_syn16(const AlphaArgs a0, const AlphaArgs a1, int half) {
+  constexpr int NT = (1 << LOGM) / 16;
+  extern __shared__ double2 dyn_lds[];
+  const bool second = (int)blockIdx.x >= half;
+  const AlphaArgs &a = second ? a1 : a0;
+  const int hi = a.hi, n = 2 * hi - 1;
+  const SynSeq us = syn_seq(a, xcd_tile(blockIdx.x - (second ? half : 0), half));
+  double2 v[16];
+  {
+    int k[8];
+    double2 z[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) k[e] = threadIdx.x + NT * e;
+    syn_gather<8>(a, us, true, k, z);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = cmulw<-1>(z[e], a.f.chirp[k[e]]);  // chirp: zero for n <= k < M
+  }
+  team16_bluestein<LOGM, -1>(a.f, dyn_lds, v);
+#pragma unroll
+  for (int r = 0; r < 8; ++r) v[r] = cmulw<-1>(v[r], a.f.chirp[threadIdx.x + NT * r]);
+  if (us.packed) {  // uniform: Z(n - k), n - k >= hi, from the thread that holds it
+    lds_barrier();
+#pragma unroll
+    for (int r = 0; r < 8; ++r) dyn_lds[lpad16(threadIdx.x + NT * r)] = v[r];
+    lds_barrier();
+  }
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const int kk = threadIdx.x + NT * r;
+    if (kk < hi) syn_store(a, us, kk, v[r], us.packed ? dyn_lds[lpad16(kk ? n - kk : 0)] : v[r]);
+  }
+}
+
 template <int LOGM, int BL>
 __global__ __launch_bounds__(kTN, 3) void k_beta_syn_t2(const BetaSynArgs a, const double2 *V1, double2 *Vt1,
                                                         const double2 *tw81, int nmt, int half) {
@@ -3070,6 +3329,142 @@ __global__ __launch_bounds__(nt_of(LOGM), occ_of(LOGM)) void k_beta_syn_h2(const
 }
 #undef S2DW_SLOTS
 
+// The same two beta stages (Bluestein, L = 2hi <= M/2) on the three-stage
+// engine, one column per workgroup.
+template <int LOGM>
+__global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_beta_ana16(const BetaAnaArgs a0, const BetaAnaArgs a1, int nmt,
+                                                                   int half) {
+  constexpr int NT = (1 << LOGM) / 16;
+  extern __shared__ double2 dyn_lds[];
+  const bool second = (int)blockIdx.x >= half;
+  const BetaAnaArgs &a = second ? a1 : a0;
+  const int hi = a.hi, L = 2 * hi, tile = xcd_tile(blockIdx.x - (second ? half : 0), half);
+  const int g = tile / nmt, m = tile - g * nmt;  // nmt = hi
+  const bool odd = (m + a.N - 1) & 1;
+  const double2 *T = a.Tg + (long long)g * hi * hi + m;
+  double2 v[16];
+  {
+    // slots k < hi in registers, slot L - k through the slots
+    double2 x[4], w[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int k = threadIdx.x + NT * r;  // < M/4, hi <= M/4
+      x[r] = T[(long long)(k < hi ? k : 0) * hi];
+      w[r] = a.tw8[k < hi ? k : 0];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int k = threadIdx.x + NT * r;
+      const double2 lo = cmulw<-1>(x[r], w[r]);
+      v[r] = odd ? make_double2(-lo.x, -lo.y) : lo;
+      if (k == 0 && odd) v[r] = make_double2(0.0, 0.0);
+      if (k < hi) dyn_lds[lpad16(k ? L - k : hi)] = k ? cmul(x[r], w[r]) : make_double2(0.0, 0.0);
+    }
+    lds_barrier();
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int k = threadIdx.x + NT * r;
+      double2 z = make_double2(0.0, 0.0);
+      if (k < hi) {
+        if (r < 4) z = v[r & 3];
+      } else if (k < L) {
+        z = dyn_lds[lpad16(k)];
+      }
+      v[r] = cmulw<-1>(z, a.f.chirp[k]);
+    }
+    lds_barrier();
+  }
+  team16_bluestein<LOGM, -1>(a.f, dyn_lds, v);
+  const double2 x0 = odd ? T[0] : make_double2(0.0, 0.0);
+  double2 *o = a.Tb + (long long)g * L * hi + m;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const int k = threadIdx.x + NT * r;
+    if (k < L) {
+      const double2 y = cmulw<-1>(v[r], a.f.chirp[k]);
+      const bool up = k >= hi;  // Tb(2n) = [x0 +] v_n, Tb(2n+1) = [x0 -] v_{L-1-n}
+      o[(long long)(up ? 2 * (L - 1 - k) + 1 : 2 * k) * hi] = up && odd ? csub(x0, y) : cadd(x0, y);
+    }
+  }
+}
+
+template <int LOGM>
+__global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_beta_syn16(const BetaSynArgs a, const double2 *V1, double2 *Vt1,
+                                                                   const double2 *tw81, int nmt, int half) {
+  constexpr int NT = (1 << LOGM) / 16;
+  extern __shared__ double2 dyn_lds[];
+  __shared__ double2 csum[NT / 64];
+  const bool second = (int)blockIdx.x >= half;
+  const double2 *tw8 = second ? tw81 : a.tw8;
+  const int hi = a.hi, L = 2 * hi, tile = xcd_tile(blockIdx.x - (second ? half : 0), half);
+  const int ni = tile / nmt, m = tile - ni * nmt;  // nmt = hi
+  const int nv = a.nval[ni], ncol = a.ncol[ni];
+  const bool odd = (m + nv) & 1;
+  const double2 *U = (second ? V1 : a.V) + (long long)ni * L * hi + m;
+  double2 v[16];
+  {
+    double2 c[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int k = threadIdx.x + NT * r;
+      const int b = k < hi ? 2 * k : 2 * (L - 1 - k) + 1;
+      v[r] = k < L ? U[(long long)b * hi] : make_double2(0.0, 0.0);
+      c[r] = a.f.chirp[k];  // zero for L <= k < M
+    }
+    double2 cs = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      cs = cadd(cs, v[r]);
+      const bool flip = odd && threadIdx.x + NT * r >= (unsigned)hi;  // odd b
+      v[r] = cmulw<-1>(flip ? make_double2(-v[r].x, -v[r].y) : v[r], c[r]);
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      cs.x += __shfl_xor(cs.x, o);
+      cs.y += __shfl_xor(cs.y, o);
+    }
+    if ((threadIdx.x & 63) == 0) csum[threadIdx.x >> 6] = cs;
+  }
+  team16_bluestein<LOGM, -1>(a.f, dyn_lds, v);  // its barriers also publish csum
+#pragma unroll
+  for (int r = 0; r < 8; ++r) v[r] = cmulw<-1>(v[r], a.f.chirp[threadIdx.x + NT * r]);
+  lds_barrier();
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const int k = threadIdx.x + NT * r;
+    if (k >= hi && k < L) dyn_lds[lpad16(k)] = v[r];
+  }
+  lds_barrier();
+  double2 *Vt = second ? Vt1 : a.Vt;
+  const int rot = ((m - nv) % 4 + 4) % 4;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int mp = threadIdx.x + NT * r;  // hi <= M/4
+    if (mp >= hi) continue;
+    double2 v3;
+    if (mp == 0) {
+      v3 = csum[0];
+#pragma unroll
+      for (int j = 1; j < NT / 64; ++j) v3 = cadd(v3, csum[j]);
+    } else {
+      const double2 w = tw8[mp];
+      v3 = cmulw<-1>(v[r], w);
+      const double2 v2m = cmul(dyn_lds[lpad16(L - mp)], w);
+      v3 = odd ? csub(v3, v2m) : cadd(v3, v2m);
+    }
+    double2 z;
+    if (rot == 0) z = v3;
+    else if (rot == 1) z = make_double2(-v3.y, v3.x);
+    else if (rot == 2) z = make_double2(-v3.x, -v3.y);
+    else z = make_double2(v3.y, -v3.x);
+    for (int kc = 0; kc < ncol; ++kc) {
+      const int c = a.col0[ni][kc];
+      const double2 o = a.cpart[ni][kc] ? make_double2(-z.y, z.x) : z;
+      Vt[((long long)c * hi + mp) * hi + m] = o;
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Grouped launches: several scales of one stage in a single grid (the two
 // full-band scales together; the small scales together).  Scale (segment) s
@@ -3165,21 +3560,21 @@ __global__ __launch_bounds__(kTN, 3) void k_alpha_c2r_gm(const SegTab t, const A
   }
 }
 
-__global__ __launch_bounds__(kTN, 3) void k_alpha_r2c_g(const SegTab t, const AlphaArgs *__restrict__ args,
+__global__ __launch_bounds__(kTN, 3) void k_alpha_syn_g(const SegTab t, const AlphaArgs *__restrict__ args,
                                                          const double *wbase) {
   __shared__ double2 lds[lpad_size(kTS)];
   const int s = seg_of(t, blockIdx.x), bid = blockIdx.x - t.first[s], nb = t.first[s + 1] - t.first[s];
   AlphaArgs a = args[s];
   a.W = const_cast<double *>(wbase) + a.woff;
   switch (t.sel[s]) {
-    S2DW_SEL(alpha_r2c_body, 5, 1, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(alpha_r2c_body, 6, 1, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(alpha_r2c_body, 7, 1, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(alpha_r2c_body, 8, 1, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(alpha_r2c_body, 9, 1, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(alpha_r2c_body, 10, 1, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(alpha_r2c_body, 11, 1, a, t.par[s], lds, bid, nb)
-    default: alpha_r2c_body<0, -1>(a, t.par[s], lds, bid, nb); break;
+    S2DW_SEL(alpha_syn_body, 5, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_syn_body, 6, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_syn_body, 7, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_syn_body, 8, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_syn_body, 9, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_syn_body, 10, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_syn_body, 11, 1, a, t.par[s], lds, bid, nb)
+    default: alpha_syn_body<0, -1>(a, t.par[s], lds, bid, nb); break;
   }
 }
 
@@ -3502,30 +3897,43 @@ TeamShape alpha_shape(const Plan *p, const FftSpec &f) {
 // work length (compile-time M folds the engine's LDS addressing into
 // immediate offsets) and on Bluestein vs direct; lengths below 32 (alpha)
 // run the generic instantiation <0, -1>, which reads both from the FftSpec.
+// Lengths of one sequence per workgroup up to 4096 slots (M = 2048: M/16 = 128
+// threads; M = 4096: 256) run on the three-stage engine.
+#define S2DW_ALPHA_CASE16(KERN, LM, ...)                                                                       \
+  case LM:                                                                                                     \
+    hipLaunchKernelGGL((KERN), g, dim3((1 << LM) / 16), lds16_of(LM), st, a0, a1, __VA_ARGS__);                \
+    break;
 #define S2DW_ALPHA_CASE(KERN, LM)                                                                              \
   case LM:                                                                                                     \
     hipLaunchKernelGGL((KERN<LM, 1>), g, dim3(nt_of(LM)), lds_of(LM), st, a0, a1, npt, half);                  \
     break;
-#define S2DW_ALPHA_LAUNCH(NAME, KERN)                                                                          \
+#define S2DW_ALPHA_LAUNCH(NAME, KERN, ...)                                                                     \
   void NAME(const TeamShape &t, const AlphaArgs &a0, const AlphaArgs &a1, int npt, int half, int blocks,       \
             hipStream_t st) {                                                                                  \
     const dim3 g(blocks);                                                                                      \
     switch (t.bl ? t.lg : 0) {                                                                                 \
       S2DW_ALPHA_CASE(KERN, 5) S2DW_ALPHA_CASE(KERN, 6) S2DW_ALPHA_CASE(KERN, 7) S2DW_ALPHA_CASE(KERN, 8)      \
-      S2DW_ALPHA_CASE(KERN, 9) S2DW_ALPHA_CASE(KERN, 10) S2DW_ALPHA_CASE(KERN, 11) S2DW_ALPHA_CASE(KERN, 12)   \
-      S2DW_ALPHA_CASE(KERN, 13)                                                                                \
+      S2DW_ALPHA_CASE(KERN, 9) S2DW_ALPHA_CASE(KERN, 10) __VA_ARGS__ S2DW_ALPHA_CASE(KERN, 13)                 \
       default: hipLaunchKernelGGL((KERN<0, -1>), g, dim3(kTN), 0, st, a0, a1, npt, half); break;               \
     }                                                                                                          \
   }
-S2DW_ALPHA_LAUNCH(launch_alpha_c2r, k_alpha_c2r_t2)
-S2DW_ALPHA_LAUNCH(launch_alpha_c2r_mom, k_alpha_c2r_t2m)
-S2DW_ALPHA_LAUNCH(launch_alpha_r2c, k_alpha_r2c_t2)
+#define S2DW_C(...) __VA_ARGS__
+constexpr int lds16_of(int lg) { return (1 << lg) * (int)sizeof(double2); }
+S2DW_ALPHA_LAUNCH(launch_alpha_c2r, k_alpha_c2r_t2, S2DW_ALPHA_CASE16(S2DW_C(k_alpha_c2r16<11, false>), 11, npt, half)
+                  S2DW_ALPHA_CASE16(S2DW_C(k_alpha_c2r16<12, false>), 12, npt, half))
+S2DW_ALPHA_LAUNCH(launch_alpha_c2r_mom, k_alpha_c2r_t2m,
+                  S2DW_ALPHA_CASE16(S2DW_C(k_alpha_c2r16<11, true>), 11, npt, half)
+                  S2DW_ALPHA_CASE16(S2DW_C(k_alpha_c2r16<12, true>), 12, npt, half))
+S2DW_ALPHA_LAUNCH(launch_alpha_syn, k_alpha_syn_t2, S2DW_ALPHA_CASE16(k_alpha_syn16<11>, 11, half)
+                  S2DW_ALPHA_CASE16(k_alpha_syn16<12>, 12, half))
+#undef S2DW_C
+#undef S2DW_ALPHA_CASE16
 #undef S2DW_ALPHA_LAUNCH
 #undef S2DW_ALPHA_CASE
 
 #define S2DW_H2_CASES(X) \
   X(4, 0) X(5, 0) X(6, 0) X(7, 0) X(8, 0) X(9, 0) X(10, 0) X(11, 0) X(4, 1) X(5, 1) X(6, 1) X(7, 1) X(8, 1) X(9, 1) \
-  X(10, 1) X(11, 1) X(12, 1) X(13, 1)
+  X(10, 1) X(13, 1)
 void launch_beta_ana(const TeamShape &t, const BetaAnaArgs &b0, const BetaAnaArgs &b1, int nmt, int half, int blocks,
                      hipStream_t st) {
   const dim3 g(blocks);
@@ -3536,6 +3944,12 @@ void launch_beta_ana(const TeamShape &t, const BetaAnaArgs &b0, const BetaAnaArg
     break;
     S2DW_H2_CASES(S2DW_X)
 #undef S2DW_X
+    case 2 * 11 + 1:
+      hipLaunchKernelGGL((k_beta_ana16<11>), g, dim3(128), lds16_of(11), st, b0, b1, nmt, half);
+      break;
+    case 2 * 12 + 1:
+      hipLaunchKernelGGL((k_beta_ana16<12>), g, dim3(256), lds16_of(12), st, b0, b1, nmt, half);
+      break;
     default: hipLaunchKernelGGL((k_beta_ana_t2<0, -1>), g, dim3(kTN), 0, st, b0, b1, nmt, half); break;
   }
 }
@@ -3550,10 +3964,24 @@ void launch_beta_syn(const TeamShape &t, const BetaSynArgs &y0, const BetaSynArg
     break;
     S2DW_H2_CASES(S2DW_X)
 #undef S2DW_X
+    case 2 * 11 + 1:
+      hipLaunchKernelGGL((k_beta_syn16<11>), g, dim3(128), lds16_of(11), st, y0, y1.V, y1.Vt, y1.tw8, nmt, half);
+      break;
+    case 2 * 12 + 1:
+      hipLaunchKernelGGL((k_beta_syn16<12>), g, dim3(256), lds16_of(12), st, y0, y1.V, y1.Vt, y1.tw8, nmt, half);
+      break;
     default: hipLaunchKernelGGL((k_beta_syn_t2<0, -1>), g, dim3(kTN), 0, st, y0, y1.V, y1.Vt, y1.tw8, nmt, half); break;
   }
 }
 #undef S2DW_H2_CASES
+// packed real rows without the gamma-DFT, for the scales whose beta stage
+// does it (gamma_first)
+void launch_alpha_r2c(const TeamShape &t, const AlphaArgs &a, int npt, int blocks, hipStream_t st) {
+  const dim3 g(blocks);
+  if (t.bl && t.lg == 12) hipLaunchKernelGGL((k_alpha_r2c_t2<12, 1>), g, dim3(nt_of(12)), lds_of(12), st, a, a, npt, blocks);
+  else if (t.bl && t.lg == 13) hipLaunchKernelGGL((k_alpha_r2c_t2<13, 1>), g, dim3(nt_of(13)), lds_of(13), st, a, a, npt, blocks);
+  else hipLaunchKernelGGL((k_alpha_r2c_t2<0, -1>), g, dim3(kTN), 0, st, a, a, npt, blocks);
+}
 
 }  // namespace
 
@@ -4170,6 +4598,13 @@ int plan_build(Plan *p, int B, int N, int J, double alpha, const double *K, cons
     if (int e = upload(d_eg, eg.data(), eg.size() * sizeof(double2), p->stream)) return e;
     p->eg = d_eg;
     p->nlist = nlist;
+    // the synthesis takes the gamma-DFT before the alpha transform wherever
+    // both its FFT stages are on the workgroup engine: the n of one parity
+    // (N + n odd) give at most the N sequences per row pair that the packed
+    // real rows take (see alpha_syn_body)
+    const auto z0 = std::find(nlist.begin(), nlist.end(), 0);
+    p->z0 = z0 == nlist.end() ? -1 : (int)(z0 - nlist.begin());
+    p->gamma_first = !nlist.empty() && N <= kMaxCol;
   }
   // LDS: the generic FFT kernels need two buffers of the work length, the
   // wave-engine kernels one 64*E region per wave.
@@ -4193,14 +4628,16 @@ int plan_build(Plan *p, int B, int N, int J, double alpha, const double *K, cons
                            (const void *)k_beta_syn_w<16>, (const void *)k_beta_syn_w<32>};
       for (const void *fn : fns) S2DW_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, maxlds));
     }
-    const void *big[] = {(const void *)k_beta_ana_h2<12, true>, (const void *)k_beta_ana_h2<13, true>,
-                         (const void *)k_beta_syn_h2<12, true>, (const void *)k_beta_syn_h2<13, true>,
-                         (const void *)k_alpha_c2r_t2<12, 1>, (const void *)k_alpha_c2r_t2<13, 1>,
-                         (const void *)k_alpha_c2r_t2m<12, 1>, (const void *)k_alpha_c2r_t2m<13, 1>,
-                         (const void *)k_alpha_r2c_t2<12, 1>, (const void *)k_alpha_r2c_t2<13, 1>};
-    for (int i = 0; i < 10; ++i)
-      if (lds_of(12 + (i & 1)) + kCsumLds <= maxlds)
-        S2DW_HIP_CHECK(hipFuncSetAttribute(big[i], hipFuncAttributeMaxDynamicSharedMemorySize, lds_of(12 + (i & 1))));
+    const struct { const void *fn; int lds; } big[] = {
+        {(const void *)k_beta_ana16<12>, lds16_of(12)},         {(const void *)k_beta_ana_h2<13, true>, lds_of(13)},
+        {(const void *)k_beta_syn16<12>, lds16_of(12)},         {(const void *)k_beta_syn_h2<13, true>, lds_of(13)},
+        {(const void *)k_alpha_c2r16<12, false>, lds16_of(12)}, {(const void *)k_alpha_c2r_t2<13, 1>, lds_of(13)},
+        {(const void *)k_alpha_c2r16<12, true>, lds16_of(12)},  {(const void *)k_alpha_c2r_t2m<13, 1>, lds_of(13)},
+        {(const void *)k_alpha_syn16<12>, lds16_of(12)},        {(const void *)k_alpha_syn_t2<13, 1>, lds_of(13)},
+        {(const void *)k_alpha_r2c_t2<12, 1>, lds_of(12)}, {(const void *)k_alpha_r2c_t2<13, 1>, lds_of(13)}};
+    for (const auto &b : big)
+      if (b.lds + kCsumLds <= maxlds)
+        S2DW_HIP_CHECK(hipFuncSetAttribute(b.fn, hipFuncAttributeMaxDynamicSharedMemorySize, b.lds));
   }
   p->d_cov = d_cov;
   p->d_Phi2 = nullptr;
@@ -4322,8 +4759,19 @@ AlphaArgs make_alpha(const Plan *p, int j, bool synthesis) {
   if (synthesis) {
     al.V = p->d_tb + s.tb_off;
     al.scale = (4.0 * (M_PI * M_PI) / (double)p->N) / (2.0 * s.hi - 1.0);
+    al.eg = p->eg;
+    al.wq = p->d_wq + p->wq_off[j];
+    al.N = p->N;
+    al.nn = (int)p->nlist.size();
+    al.z0 = p->z0;
   }
   return al;
+}
+
+// workgroups of a synthesis alpha launch over one scale (alpha_syn_body)
+int syn_blocks(const Plan *p, int hi, int per) {
+  const int q = hi * (2 * (int)p->nlist.size() - (p->z0 >= 0));
+  return (q + per - 1) / per;
 }
 
 BetaSynArgs make_beta_syn(const Plan *p, int j) {
@@ -4363,12 +4811,11 @@ int beta_sel(const TeamShape &t) { return t.h2 ? kSelH2 + 2 * t.lg + t.bl : 0; }
 // Grouped launches (all on the workgroup FFT engine): the two full-band
 // scales j = 0, 1 (same shapes) in one launch per stage on the main stream,
 // and the small scales j >= 2 in one launch per stage on the helper stream:
-// analysis beta + alpha c2r, synthesis alpha r2c + gamma + beta.  Segment
+// analysis beta + alpha c2r, synthesis alpha (with the gamma-DFT) + beta.  Segment
 // tables go in the kernel arguments, the stage arguments in device tables.
 struct Group {
   bool ana = false, syn = false;
   SegTab ba{}, ac{}, ar{}, bs{};
-  GammaTab gm{};
   BetaAnaArgs *d_ba = nullptr;
   AlphaArgs *d_ac = nullptr, *d_ar = nullptr;
   BetaSynArgs *d_bs = nullptr;
@@ -4377,7 +4824,6 @@ struct Group {
 struct GroupState {
   Group g[2];                        // 1: scales 2..J, or 0..J on one stream (0 unused)
   std::vector<char> in_ana, in_syn;  // per scale: runs in a group
-  int nmax = 8;
   bool pair = false;                 // scales 0 and 1 run as pair launches
 };
 
@@ -4397,7 +4843,7 @@ int build_group(Plan *p, GroupState *gs, int gi, int j0, int j1) {
   std::vector<BetaSynArgs> bs;
   std::vector<int> taken;
   bool ok = j1 - j0 >= 2 || (gi == 1 && j1 > j0);
-  const bool syn_ok = nn > 0 && N <= kMaxCol;
+  const bool syn_ok = p->gamma_first;
   for (int j = j0; j < j1 && ok; ++j) {
     const Scale &s = p->sc[j];
     if (scale_empty(s)) {
@@ -4425,11 +4871,8 @@ int build_group(Plan *p, GroupState *gs, int gi, int j0, int j1) {
     add(G.ba, nmt * N, beta_sel(tb), nmt);
     add(G.bs, nmt * nn, beta_sel(tb), nmt);
     add(G.ac, npt * N, alpha_sel(ta), npt);
-    add(G.ar, npt * N, alpha_sel(ta), npt);
+    add(G.ar, syn_blocks(p, s.hi, ta.per), alpha_sel(ta), 0);
     taken.push_back(j);
-    const int gj = G.gm.nseg++;
-    G.gm.first[gj + 1] = G.gm.first[gj] + (int)((2LL * s.hi * s.hi + 255) / 256);
-    G.gm.g[gj] = GammaSeg{p->d_tb + s.tb_off, p->d_wq + p->wq_off[j], s.hi};
     ba.push_back(b);
     a.moff = 8 * p->momf_rec0[j];
     ac.push_back(a);
@@ -4468,7 +4911,6 @@ int build_groups(Plan *p) {
   p->groups = gs;
   gs->in_ana.assign(Jp1, 0);
   gs->in_syn.assign(Jp1, 0);
-  gs->nmax = N <= 8 ? 8 : N <= 16 ? 16 : 32;
   // moments records of the analysis that reduces instead of storing: one
   // per alpha-c2r workgroup, scales in order
   p->momf_rec0.assign(Jp1 + 1, 0);
@@ -4848,29 +5290,17 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
   }
   const GroupState *grp = static_cast<const GroupState *>(p->groups);
   const int nn_all = (int)p->nlist.size();
-  const bool pair = grp && grp->pair && nn_all > 0 && N <= kMaxCol;
-  // plans on one stream run the gamma-DFT of the small scales and of the
-  // pair as one launch (one segment table), after both alpha stages
-  const bool gmerge = p->single_stream && pair && grp->g[1].syn && grp->g[1].gm.nseg + 2 <= kMaxSc;
-  auto launch_gamma = [&](const GammaTab &t, hipStream_t sq) {
-    const dim3 gg(t.first[t.nseg]);
-    if (N <= 8) hipLaunchKernelGGL(k_gamma_syn_g<8>, gg, dim3(256), 0, sq, t, N, nn_all, p->eg);
-    else if (N <= 16) hipLaunchKernelGGL(k_gamma_syn_g<16>, gg, dim3(256), 0, sq, t, N, nn_all, p->eg);
-    else hipLaunchKernelGGL(k_gamma_syn_g<32>, gg, dim3(256), 0, sq, t, N, nn_all, p->eg);
-  };
+  const bool pair = grp && grp->pair && p->gamma_first;
   for (int gi = 1; gi >= 0; --gi) {
     if (!grp || !grp->g[gi].syn) continue;
     const Group &G = grp->g[gi];
     hipStream_t sg = (conc && gi == 1) ? p->aux : st;
     {
       StageTimer tm(p, 10);
-      hipLaunchKernelGGL(k_alpha_r2c_g, dim3(G.ar.first[G.ar.nseg]), dim3(kTN), 0, sg, G.ar, G.d_ar, d_wav);
+      hipLaunchKernelGGL(k_alpha_syn_g, dim3(G.ar.first[G.ar.nseg]), dim3(kTN), 0, sg, G.ar, G.d_ar, d_wav);
       S2DW_HIP_CHECK(hipGetLastError());
     }
-    if (gmerge) continue;  // gamma and beta after the pair's alpha
     StageTimer tm(p, 10);
-    launch_gamma(G.gm, sg);
-    S2DW_HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL(k_beta_syn_g, dim3(G.bs.first[G.bs.nseg]), dim3(kTN), 0, sg, G.bs, G.d_bs);
     S2DW_HIP_CHECK(hipGetLastError());
   }
@@ -4880,34 +5310,16 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
     a0.logT = a1.logT = team_logTw(p, a0.f, false);
     a0.W = const_cast<double *>(d_wav + p->sc[0].wav_off);
     a1.W = const_cast<double *>(d_wav + p->sc[1].wav_off);
-    const int npt = (a0.hi + ta.per - 1) / ta.per;
     {
       StageTimer tm(p, 5);
-      if (p->d_otw) {
-        const int npo = (kOddHi + kOddT - 1) / kOddT;
-        hipLaunchKernelGGL((k_alpha_r2c_o2<31, 11, 3>), dim3(2 * npo * N), dim3(kOddNT), 0, st, a0, a1, npo, p->d_otw);
-      } else {
-        launch_alpha_r2c(ta, a0, a1, npt, npt * N, 2 * npt * N, st);
-      }
+      const int nb = syn_blocks(p, a0.hi, p->d_otw ? 1 : ta.per);
+      if (p->d_otw)
+        hipLaunchKernelGGL((k_alpha_syn_o2<31, 11, 3>), dim3(2 * nb), dim3(kOddNT), 0, st, a0, a1, p->d_otw);
+      else
+        launch_alpha_syn(ta, a0, a1, 0, nb, 2 * nb, st);
       S2DW_HIP_CHECK(hipGetLastError());
     }
     StageTimer tm(p, 6);
-    // the pair's segments, after the small scales' when merged
-    GammaTab gt = gmerge ? grp->g[1].gm : GammaTab{};
-    const int s0 = gmerge ? gt.nseg : 0;
-    for (int j = 0; j < 2; ++j) {
-      const Scale &s = p->sc[j];
-      gt.g[s0 + j] = GammaSeg{p->d_tb + s.tb_off, p->d_wq + p->wq_off[j], s.hi};
-      gt.first[s0 + j + 1] = gt.first[s0 + j] + (int)((2LL * s.hi * s.hi + 255) / 256);
-    }
-    gt.nseg = s0 + 2;
-    launch_gamma(gt, st);
-    S2DW_HIP_CHECK(hipGetLastError());
-    if (gmerge) {
-      const Group &G = grp->g[1];
-      hipLaunchKernelGGL(k_beta_syn_g, dim3(G.bs.first[G.bs.nseg]), dim3(kTN), 0, st, G.bs, G.d_bs);
-      S2DW_HIP_CHECK(hipGetLastError());
-    }
     BetaSynArgs y0 = make_beta_syn(p, 0), y1 = make_beta_syn(p, 1);
     const TeamShape tb = beta_shape(p, y0.f, y0.hi);
     y0.logT = y1.logT = team_logTw(p, y0.f, true);
@@ -4920,22 +5332,23 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
     if ((grp && grp->in_syn[j]) || (pair && j < 2)) continue;
     hipStream_t sj = (conc && j >= 2) ? p->aux : st;
     if (scale_empty(s)) continue;
-    // alpha r2c -> V (tb buffer)
+    BetaSynArgs b = make_beta_syn(p, j);
+    const TeamShape tb = beta_shape(p, b.f, s.hi);
+    const bool team_beta = nn_all > 0 && tb.lg >= 0 && N <= kMaxCol;
+    bool gamma_done = false;
+    // alpha r2c -> V, or with the gamma-DFT -> U (tb buffer)
     {
       StageTimer tm(p, 5);
-      AlphaArgs al{};
-      al.f = p->ffts[s.fa];
-      al.logT = fft_logT(al.f, 4);
-      al.hi = s.hi;
+      AlphaArgs al = make_alpha(p, j, true);
       al.W = const_cast<double *>(d_wav + s.wav_off);
-      al.V = p->d_tb + s.tb_off;
-      al.scale = (4.0 * (M_PI * M_PI) / (double)N) / (2.0 * s.hi - 1.0);
       const WaveShape ws = wave_shape(p, al.f);
       const TeamShape ts = alpha_shape(p, al.f);
       if (ts.lg >= 0) {
         al.logT = team_logTw(p, al.f, false);
-        const int npt = (s.hi + ts.per - 1) / ts.per;
-        launch_alpha_r2c(ts, al, al, npt, npt * N, npt * N, sj);
+        gamma_done = team_beta && p->gamma_first;
+        const int npt = (s.hi + ts.per - 1) / ts.per, nb = syn_blocks(p, s.hi, ts.per);
+        if (gamma_done) launch_alpha_syn(ts, al, al, 0, nb, nb, sj);
+        else launch_alpha_r2c(ts, al, npt, npt * N, sj);
       } else if (ws.ok) {
         al.logT = ws.logTw;
         const int per = ws.WPB << ws.logTw;
@@ -4952,41 +5365,20 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
     // beta -> Vt (tg buffer)
     {
       StageTimer tm(p, 6);
-      BetaSynArgs b{};
-      b.f = p->ffts[s.fb];
-      b.logT = fft_logT(b.f, 4);
-      b.hi = s.hi;
-      b.N = N;
-      b.NCtot = NCs;
-      b.V = p->d_tb + s.tb_off;
-      b.wq = p->d_wq + p->wq_off[j];
-      b.tw8 = p->d_tw8 + p->tw8_off[j];
-      b.eg = p->eg;
-      b.Vt = p->d_tg + s.tg_off;
-      const int nn = (int)p->nlist.size();
-      for (int i = 0; i < nn; ++i) {
-        b.nval[i] = p->nlist[i];
-        b.ncol[i] = 0;
-        for (int c = 0; c < NCs; ++c)
-          if (p->cols_s[c].n == p->nlist[i]) {
-            b.col0[i][b.ncol[i]] = c;
-            b.cpart[i][b.ncol[i]] = p->cols_s[c].part;
-            ++b.ncol[i];
-          }
-      }
+      const int nn = nn_all;
       const WaveShape ws = wave_shape(p, b.f);
-      const TeamShape ts = beta_shape(p, b.f, s.hi);
-      if (nn > 0 && ts.lg >= 0 && N <= kMaxCol) {
-        const long long plane = 2LL * s.hi * s.hi;
-        const dim3 gg((unsigned)((plane + 255) / 256));
-        double2 *Vj = p->d_tb + s.tb_off;
-        if (N <= 8) hipLaunchKernelGGL(k_gamma_syn<8>, gg, dim3(256), 0, sj, Vj, s.hi, N, nn, b.wq, b.eg);
-        else if (N <= 16) hipLaunchKernelGGL(k_gamma_syn<16>, gg, dim3(256), 0, sj, Vj, s.hi, N, nn, b.wq, b.eg);
-        else hipLaunchKernelGGL(k_gamma_syn<32>, gg, dim3(256), 0, sj, Vj, s.hi, N, nn, b.wq, b.eg);
-        S2DW_HIP_CHECK(hipGetLastError());
+      if (team_beta) {
+        if (!gamma_done) {
+          const dim3 gg((unsigned)((2LL * s.hi * s.hi + 255) / 256));
+          double2 *Vj = p->d_tb + s.tb_off;
+          if (N <= 8) hipLaunchKernelGGL(k_gamma_syn<8>, gg, dim3(256), 0, sj, Vj, s.hi, N, nn, b.wq, b.eg);
+          else if (N <= 16) hipLaunchKernelGGL(k_gamma_syn<16>, gg, dim3(256), 0, sj, Vj, s.hi, N, nn, b.wq, b.eg);
+          else hipLaunchKernelGGL(k_gamma_syn<32>, gg, dim3(256), 0, sj, Vj, s.hi, N, nn, b.wq, b.eg);
+          S2DW_HIP_CHECK(hipGetLastError());
+        }
         b.logT = team_logTw(p, b.f, true);
-        const int nmt = (s.hi + ts.per - 1) / ts.per;
-        launch_beta_syn(ts, b, b, nmt, nmt * nn, nmt * nn, sj);
+        const int nmt = (s.hi + tb.per - 1) / tb.per;
+        launch_beta_syn(tb, b, b, nmt, nmt * nn, nmt * nn, sj);
         S2DW_HIP_CHECK(hipGetLastError());
       } else if (nn > 0 && ws.ok) {
         b.logT = ws.logTw;
