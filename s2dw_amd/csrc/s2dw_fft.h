@@ -772,11 +772,12 @@ __device__ __forceinline__ void team_fft_core(const FftSpec &s, double2 *buf, in
 // radix-8 engine of 512 threads writes and reads them eight times each and
 // spills (its four stages of twiddles stay in registers: 128 of 128 VGPRs;
 // here 2 waves per SIMD leave 256).
-// Physical slot of logical slot i: i ^ ((i >> 4) & 15); consecutive slots and
-// slots 16 apart, the two patterns of the stages, both fall in distinct
-// 16-byte bank groups over 16 lanes.
+// Physical slot of logical slot i: i + i/16.  Consecutive slots and slots 8 or
+// 16 apart, the patterns of the stages, fall in distinct banks over 16 lanes,
+// and every stage's slots are one base per thread plus compile-time offsets
+// (with an xor swizzle the 16 addresses of a stage took registers and spilled).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int lpad16(int i) { return i ^ ((i >> 4) & 15); }
+__host__ __device__ constexpr int lpad16(int i) { return i + (i >> 4); }
 
 // v[r] *= w^r (sign of DIR), r = 1..15, from w, w^2, w^4, w^8
 template <int DIR>
@@ -819,40 +820,50 @@ __device__ __forceinline__ void dft16_half(double2 *v) {
   }
 }
 
+// One exchange of the 16 values of every thread through M padded doubles of LDS, the
+// real parts and then the imaginary parts: half the LDS of whole values, so
+// that three workgroups of M = 4096 share a CU instead of two.  wr(r), rd(r):
+// slots written and read.  The slots may be written again after a barrier.
+template <typename Wr, typename Rd>
+__device__ __forceinline__ void exchange16(double *buf, double2 (&v)[16], Wr wr, Rd rd) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) buf[wr(r)] = v[r].x;
+  lds_barrier();
+#pragma unroll
+  for (int r = 0; r < 16; ++r) v[r].x = buf[rd(r)];
+  lds_barrier();
+#pragma unroll
+  for (int r = 0; r < 16; ++r) buf[wr(r)] = v[r].y;
+  lds_barrier();
+#pragma unroll
+  for (int r = 0; r < 16; ++r) v[r].y = buf[rd(r)];
+}
+
 // In: v[r], r < 8 = input k = threadIdx.x + NT r times chirp_k^{DIR} (zero for
 // k >= n; k >= M/2 is zero).  Out: v[r] = convolution output k = threadIdx.x
-// + NT r, to be multiplied by chirp_k^{DIR} (k < n <= M/2, so r < 8).  The
-// slots may be reused after a barrier.
+// + NT r, to be multiplied by chirp_k^{DIR} (k < n <= M/2, so r < 8).  buf:
+// lpad16(M) doubles, free again after a barrier.
 template <int LOGM, int DIR>
-__device__ __forceinline__ void team16_bluestein(const FftSpec &s, double2 *buf, double2 (&v)[16]) {
+__device__ __forceinline__ void team16_bluestein(const FftSpec &s, double *buf, double2 (&v)[16]) {
   constexpr int M = 1 << LOGM, NT = M / 16, R3 = M / 256, NC = 16 / R3;
   static_assert(R3 == 16 || R3 == 8, "M = 4096 or 2048");
   const double2 *__restrict__ tw = s.tw;
   const double2 *__restrict__ F = DIR > 0 ? s.filt_b : s.filt_f;
   // forward, Ns = 1
   dft16_half<-1>(v);
-  {
-    const int tid = stage_tid();
-#pragma unroll
-    for (int r = 0; r < 16; ++r) buf[lpad16(16 * tid + r)] = v[r];
-  }
-  lds_barrier();
   // forward, Ns = 16
   {
     const int tid = stage_tid(), jm = tid & 15, e = jm * (M / 256);
     const double2 w1 = tw[e], w2 = tw[2 * e], w4 = tw[4 * e], w8 = tw[8 * e];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = buf[lpad16(tid + NT * r)];
-    lds_barrier();
+    const int wb = 17 * tid, rb = lpad16(tid);
+    exchange16(buf, v, [=](int r) { return wb + r; }, [=](int r) { return rb + lpad16(NT * r); });
     twiddle16<-1>(v, w1, w2, w4, w8);
     dft16<-1>(v);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) buf[lpad16((tid - jm) * 16 + jm + 16 * r)] = v[r];
   }
   lds_barrier();
   // forward, Ns = 256 (radix R3), the filter, and backward, Ns = 1 (radix R3)
   {
-    const int tid = stage_tid();
+    const int tid = stage_tid(), jm = tid & 15;
     double2 f[16], w1[NC], w2[NC], w4[NC], w8[NC];
 #pragma unroll
     for (int q = 0; q < NC; ++q) {
@@ -861,23 +872,28 @@ __device__ __forceinline__ void team16_bluestein(const FftSpec &s, double2 *buf,
       w2[q] = tw[2 * jj];
       w4[q] = tw[4 * jj];
       w8[q] = R3 == 16 ? tw[8 * jj] : w4[q];
-#pragma unroll
-      for (int r = 0; r < R3; ++r) v[q * R3 + r] = buf[lpad16(jj + 256 * r)];
-#pragma unroll
-      for (int r = 0; r < R3; ++r) f[q * R3 + r] = F[jj + 256 * r];
     }
-    lds_barrier();
+    const int wb = (tid - jm) * 17 + jm, rb = lpad16(tid);
+    exchange16(buf, v, [=](int r) { return wb + 17 * r; },
+               [=](int r) { return rb + lpad16(NT * (r / R3) + 256 * (r % R3)); });
 #pragma unroll
     for (int q = 0; q < NC; ++q) {
       double2 *x = v + q * R3;
       if constexpr (R3 == 16) twiddle16<-1>(x, w1[q], w2[q], w4[q], w8[q]);
       else twiddle_powers<R3, -1>(x, w1[q], w2[q], w4[q], w8[q]);
+    }
+    // the filter is loaded after the twiddles: in flight earlier it makes the
+    // 168 registers of three waves per SIMD spill
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) f[r] = F[tid + NT * (r / R3) + 256 * (r % R3)];
+#pragma unroll
+    for (int q = 0; q < NC; ++q) {
+      double2 *x = v + q * R3;
       dft_pow2<R3, -1>(x);
 #pragma unroll
       for (int r = 0; r < R3; ++r) x[r] = cmul(x[r], f[q * R3 + r]);
       dft_pow2<R3, +1>(x);
-#pragma unroll
-      for (int r = 0; r < R3; ++r) buf[lpad16((tid + NT * q) * R3 + r)] = x[r];
     }
   }
   lds_barrier();
@@ -885,21 +901,19 @@ __device__ __forceinline__ void team16_bluestein(const FftSpec &s, double2 *buf,
   {
     const int tid = stage_tid(), jm = tid & (R3 - 1), e = jm * 16;
     const double2 w1 = tw[e], w2 = tw[2 * e], w4 = tw[4 * e], w8 = tw[8 * e];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = buf[lpad16(tid + NT * r)];
-    lds_barrier();
+    const int wb = lpad16(R3 * tid), rb = lpad16(tid);  // R3 tid mod 16 + r mod R3 < 16
+    exchange16(buf, v, [=](int r) { return wb + lpad16(NT * R3 * (r / R3)) + r % R3; },
+               [=](int r) { return rb + lpad16(NT * r); });
     twiddle16<+1>(v, w1, w2, w4, w8);
     dft16<+1>(v);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) buf[lpad16((tid - jm) * 16 + jm + R3 * r)] = v[r];
   }
   lds_barrier();
   // backward, Ns = M/16
   {
-    const int tid = stage_tid();
+    const int tid = stage_tid(), jm = tid & (R3 - 1);
     const double2 w1 = tw[tid], w2 = tw[2 * tid], w4 = tw[4 * tid], w8 = tw[8 * tid];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = buf[lpad16(tid + NT * r)];
+    const int wb = (tid - jm) * 17 + jm, rb = lpad16(tid);  // jm + R3 r mod 16 < 16
+    exchange16(buf, v, [=](int r) { return wb + lpad16(R3 * r); }, [=](int r) { return rb + lpad16(NT * r); });
     twiddle16<+1>(v, w1, w2, w4, w8);
     dft16<+1>(v);
   }

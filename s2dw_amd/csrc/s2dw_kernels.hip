@@ -3035,7 +3035,7 @@ __global__ __launch_bounds__(NT, 3) void k_alpha_syn_o2(const AlphaArgs a0, cons
 // (the mirrored halves of the packed rows and of the beta columns).
 // ---------------------------------------------------------------------------
 template <int LOGM, bool MOM>
-__global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_alpha_c2r16(const AlphaArgs a0, const AlphaArgs a1, int npt,
+__global__ __launch_bounds__((1 << LOGM) / 16, MOM && LOGM == 12 ? 2 : 3) void k_alpha_c2r16(const AlphaArgs a0, const AlphaArgs a1, int npt,
                                                                     int half) {
   constexpr int NT = (1 << LOGM) / 16;
   extern __shared__ double2 dyn_lds[];
@@ -3063,7 +3063,7 @@ __global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_alpha_c2r16(const Alpha
       v[r] = k < n ? cmulw<+1>(z, c[r]) : make_double2(0.0, 0.0);
     }
   }
-  team16_bluestein<LOGM, +1>(a.f, dyn_lds, v);
+  team16_bluestein<LOGM, +1>(a.f, (double *)dyn_lds, v);
   if constexpr (MOM) {
     double x[16], wt[16];
 #pragma unroll
@@ -3090,7 +3090,7 @@ __global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_alpha_c2r16(const Alpha
 }
 
 template <int LOGM>
-__global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_alpha_syn16(const AlphaArgs a0, const AlphaArgs a1, int half) {
+__global__ __launch_bounds__((1 << LOGM) / 16, 3) void k_alpha_syn16(const AlphaArgs a0, const AlphaArgs a1, int half) {
   constexpr int NT = (1 << LOGM) / 16;
   extern __shared__ double2 dyn_lds[];
   const bool second = (int)blockIdx.x >= half;
@@ -3107,19 +3107,22 @@ __global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_alpha_syn16(const Alpha
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = cmulw<-1>(z[e], a.f.chirp[k[e]]);  // chirp: zero for n <= k < M
   }
-  team16_bluestein<LOGM, -1>(a.f, dyn_lds, v);
+  team16_bluestein<LOGM, -1>(a.f, (double *)dyn_lds, v);
 #pragma unroll
   for (int r = 0; r < 8; ++r) v[r] = cmulw<-1>(v[r], a.f.chirp[threadIdx.x + NT * r]);
   if (us.packed) {  // uniform: Z(n - k), n - k >= hi, from the thread that holds it
     lds_barrier();
 #pragma unroll
-    for (int r = 0; r < 8; ++r) dyn_lds[lpad16(threadIdx.x + NT * r)] = v[r];
+    for (int r = 0; r < 8; ++r) {
+      const int k = threadIdx.x + NT * r;
+      if (k >= hi && k < n) dyn_lds[k - hi] = v[r];
+    }
     lds_barrier();
   }
 #pragma unroll
   for (int r = 0; r < 8; ++r) {
     const int kk = threadIdx.x + NT * r;
-    if (kk < hi) syn_store(a, us, kk, v[r], us.packed ? dyn_lds[lpad16(kk ? n - kk : 0)] : v[r]);
+    if (kk < hi) syn_store(a, us, kk, v[r], us.packed && kk ? dyn_lds[n - kk - hi] : v[r]);
   }
 }
 
@@ -3332,7 +3335,7 @@ __global__ __launch_bounds__(nt_of(LOGM), occ_of(LOGM)) void k_beta_syn_h2(const
 // The same two beta stages (Bluestein, L = 2hi <= M/2) on the three-stage
 // engine, one column per workgroup.
 template <int LOGM>
-__global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_beta_ana16(const BetaAnaArgs a0, const BetaAnaArgs a1, int nmt,
+__global__ __launch_bounds__((1 << LOGM) / 16, 3) void k_beta_ana16(const BetaAnaArgs a0, const BetaAnaArgs a1, int nmt,
                                                                    int half) {
   constexpr int NT = (1 << LOGM) / 16;
   extern __shared__ double2 dyn_lds[];
@@ -3358,7 +3361,7 @@ __global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_beta_ana16(const BetaAn
       const double2 lo = cmulw<-1>(x[r], w[r]);
       v[r] = odd ? make_double2(-lo.x, -lo.y) : lo;
       if (k == 0 && odd) v[r] = make_double2(0.0, 0.0);
-      if (k < hi) dyn_lds[lpad16(k ? L - k : hi)] = k ? cmul(x[r], w[r]) : make_double2(0.0, 0.0);
+      if (k < hi) dyn_lds[k ? hi - k : 0] = k ? cmul(x[r], w[r]) : make_double2(0.0, 0.0);
     }
     lds_barrier();
 #pragma unroll
@@ -3368,13 +3371,13 @@ __global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_beta_ana16(const BetaAn
       if (k < hi) {
         if (r < 4) z = v[r & 3];
       } else if (k < L) {
-        z = dyn_lds[lpad16(k)];
+        z = dyn_lds[k - hi];
       }
       v[r] = cmulw<-1>(z, a.f.chirp[k]);
     }
     lds_barrier();
   }
-  team16_bluestein<LOGM, -1>(a.f, dyn_lds, v);
+  team16_bluestein<LOGM, -1>(a.f, (double *)dyn_lds, v);
   const double2 x0 = odd ? T[0] : make_double2(0.0, 0.0);
   double2 *o = a.Tb + (long long)g * L * hi + m;
 #pragma unroll
@@ -3389,7 +3392,7 @@ __global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_beta_ana16(const BetaAn
 }
 
 template <int LOGM>
-__global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_beta_syn16(const BetaSynArgs a, const double2 *V1, double2 *Vt1,
+__global__ __launch_bounds__((1 << LOGM) / 16, 3) void k_beta_syn16(const BetaSynArgs a, const double2 *V1, double2 *Vt1,
                                                                    const double2 *tw81, int nmt, int half) {
   constexpr int NT = (1 << LOGM) / 16;
   extern __shared__ double2 dyn_lds[];
@@ -3425,14 +3428,14 @@ __global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_beta_syn16(const BetaSy
     }
     if ((threadIdx.x & 63) == 0) csum[threadIdx.x >> 6] = cs;
   }
-  team16_bluestein<LOGM, -1>(a.f, dyn_lds, v);  // its barriers also publish csum
+  team16_bluestein<LOGM, -1>(a.f, (double *)dyn_lds, v);  // its barriers also publish csum
 #pragma unroll
   for (int r = 0; r < 8; ++r) v[r] = cmulw<-1>(v[r], a.f.chirp[threadIdx.x + NT * r]);
   lds_barrier();
 #pragma unroll
   for (int r = 0; r < 8; ++r) {
     const int k = threadIdx.x + NT * r;
-    if (k >= hi && k < L) dyn_lds[lpad16(k)] = v[r];
+    if (k >= hi && k < L) dyn_lds[k - hi] = v[r];
   }
   lds_barrier();
   double2 *Vt = second ? Vt1 : a.Vt;
@@ -3449,7 +3452,7 @@ __global__ __launch_bounds__((1 << LOGM) / 16, 2) void k_beta_syn16(const BetaSy
     } else {
       const double2 w = tw8[mp];
       v3 = cmulw<-1>(v[r], w);
-      const double2 v2m = cmul(dyn_lds[lpad16(L - mp)], w);
+      const double2 v2m = cmul(dyn_lds[hi - mp], w);
       v3 = odd ? csub(v3, v2m) : cadd(v3, v2m);
     }
     double2 z;
@@ -3918,7 +3921,7 @@ TeamShape alpha_shape(const Plan *p, const FftSpec &f) {
     }                                                                                                          \
   }
 #define S2DW_C(...) __VA_ARGS__
-constexpr int lds16_of(int lg) { return (1 << lg) * (int)sizeof(double2); }
+constexpr int lds16_of(int lg) { return lpad16(1 << lg) * (int)sizeof(double); }
 S2DW_ALPHA_LAUNCH(launch_alpha_c2r, k_alpha_c2r_t2, S2DW_ALPHA_CASE16(S2DW_C(k_alpha_c2r16<11, false>), 11, npt, half)
                   S2DW_ALPHA_CASE16(S2DW_C(k_alpha_c2r16<12, false>), 12, npt, half))
 S2DW_ALPHA_LAUNCH(launch_alpha_c2r_mom, k_alpha_c2r_t2m,
