@@ -1864,7 +1864,8 @@ struct BetaAnaArgs {
   FftSpec f;
   int hi, N, logT;
   const double2 *Tg;
-  double2 *Tb;
+  double2 *Tb;        // [g][m][b], or [g][b][m] in the reference-rounding form: strides tbb, tbm
+  int tbb, tbm;
   const double2 *tw8;
 };
 
@@ -1892,7 +1893,7 @@ __global__ __launch_bounds__(256) void k_beta_ana(const BetaAnaArgs a) {
   const double2 *out = fft_exec<+1>(a.f, A, Bf, a.logT);
   for (int idx = threadIdx.x; idx < (hi << a.logT); idx += blockDim.x) {
     const int t = idx & (T - 1), bp = idx >> a.logT, m = m0 + t;
-    if (m < hi) a.Tb[((long long)g * n + 2 * bp + r) * hi + m] = out[idx];
+    if (m < hi) a.Tb[(long long)g * n * hi + (long long)(2 * bp + r) * a.tbb + (long long)m * a.tbm] = out[idx];
   }
 }
 
@@ -1903,7 +1904,8 @@ __global__ __launch_bounds__(256) void k_beta_ana(const BetaAnaArgs a) {
 struct AlphaArgs {
   FftSpec f;
   int hi, logT;
-  const double2 *Tb;  // analysis input / synthesis output [g][b][m]
+  const double2 *Tb;  // analysis input, [g][m][b] (BetaAnaArgs): strides tbb, tbm
+  int tbb, tbm;
   double *W;          // per-scale wav [g][b][a]
   double2 *V;         // synthesis output
   double scale;       // synthesis scaling
@@ -1922,18 +1924,19 @@ __global__ __launch_bounds__(256) void k_alpha_c2r(const AlphaArgs a) {
   const int g = blockIdx.y;
   for (int t = 0; t < T; ++t) {
     const int pidx = blockIdx.x * T + t;
-    const double2 *rb = a.Tb + ((long long)g * 2 * hi + 2 * pidx) * hi;
-    const double2 *rb1 = rb + hi;
+    const double2 *rb = a.Tb + (long long)g * 2 * hi * hi + (long long)(2 * pidx) * a.tbb;
+    const double2 *rb1 = rb + a.tbb;
+    const long long sm = a.tbm;
     for (int k = threadIdx.x; k < n; k += blockDim.x) {
       double2 z = make_double2(0.0, 0.0);
       if (pidx < hi) {
         if (k == 0) {
           z = make_double2(rb[0].x, rb1[0].x);
         } else if (k < hi) {
-          const double2 p = rb[k], q = rb1[k];
+          const double2 p = rb[k * sm], q = rb1[k * sm];
           z = make_double2(p.x - q.y, p.y + q.x);
         } else {
-          const double2 p = rb[n - k], q = rb1[n - k];
+          const double2 p = rb[(n - k) * sm], q = rb1[(n - k) * sm];
           z = make_double2(p.x + q.y, -p.y + q.x);
         }
       }
@@ -2098,7 +2101,8 @@ __global__ __launch_bounds__(512 / (E / 16)) void k_beta_ana_w(const BetaAnaArgs
   __syncthreads();
   for (int idx = threadIdx.x; idx < hi * TMW; idx += blockDim.x) {
     const int t = idx % TMW, bp = idx / TMW, m = m0 + t;
-    if (m < hi) a.Tb[((long long)g * n + 2 * bp + r) * hi + m] = lds[(t >> logTw) * (64 * E) + (bp << logTw) + (t & (Tw - 1))];
+    if (m < hi)
+      a.Tb[(long long)g * n * hi + (long long)(2 * bp + r) * a.tbb + (long long)m * a.tbm] = lds[(t >> logTw) * (64 * E) + (bp << logTw) + (t & (Tw - 1))];
   }
 }
 
@@ -2114,18 +2118,19 @@ __global__ __launch_bounds__(512 / (E / 16)) void k_alpha_c2r_w(const AlphaArgs 
   const int p0 = (blockIdx.x * WPB + w) * Tw;
   for (int t = 0; t < Tw; ++t) {
     const int pidx = p0 + t;
-    const double2 *rb = a.Tb + ((long long)g * 2 * hi + 2 * pidx) * hi;
-    const double2 *rb1 = rb + hi;
+    const double2 *rb = a.Tb + (long long)g * 2 * hi * hi + (long long)(2 * pidx) * a.tbb;
+    const double2 *rb1 = rb + a.tbb;
+    const long long sm = a.tbm;
     for (int k = lane; k < n; k += 64) {
       double2 z = make_double2(0.0, 0.0);
       if (pidx < hi) {
         if (k == 0) {
           z = make_double2(rb[0].x, rb1[0].x);
         } else if (k < hi) {
-          const double2 p = rb[k], q = rb1[k];
+          const double2 p = rb[k * sm], q = rb1[k * sm];
           z = make_double2(p.x - q.y, p.y + q.x);
         } else {
-          const double2 p = rb[n - k], q = rb1[n - k];
+          const double2 p = rb[(n - k) * sm], q = rb1[(n - k) * sm];
           z = make_double2(p.x + q.y, -p.y + q.x);
         }
       }
@@ -2311,10 +2316,29 @@ __device__ __forceinline__ void beta_ana_body(const BetaAnaArgs &a, int nmt, dou
     if (m < hi && bp < hi) {
       double2 y = lds[lpad((bp << logTw) + 2 * mc + r)];
       if (bluestein) y = cmulw<+1>(y, f.chirp[bp]);
-      a.Tb[((long long)g * n + 2 * bp + r) * hi + m] = y;
+      a.Tb[(long long)g * n * hi + (2 * bp + r) * a.tbb + m * a.tbm] = y;
     }
   }
   (void)M;
+}
+
+// Rows p = rb, q = rb + sb of a packed pair at the lane's own k: lanes 2i and
+// 2i + 1 (both active) load p and q of the even lane's k = ke and then of the
+// odd lane's k = ko, side by side in memory where sb = 1, and swap halves.
+__device__ __forceinline__ double swap1(double v) {  // the value of lane ^ 1
+  int2 x = __builtin_bit_cast(int2, v);
+  x.x = __builtin_amdgcn_update_dpp(0, x.x, 0xB1, 0xF, 0xF, true);
+  x.y = __builtin_amdgcn_update_dpp(0, x.y, 0xB1, 0xF, 0xF, true);
+  return __builtin_bit_cast(double, x);
+}
+__device__ __forceinline__ void load_pair(const double2 *rb, int sb, int sm, int ke, int ko, double2 &p, double2 &q) {
+  const bool odd = threadIdx.x & 1;
+  const double2 *c = rb + (odd ? sb : 0);
+  const double2 r1 = c[ke * sm], r2 = c[ko * sm];  // < 2 hi^2 < 2^31
+  const double2 snd = odd ? r1 : r2;
+  const double2 rcv = make_double2(swap1(snd.x), swap1(snd.y));
+  p = odd ? rcv : r1;
+  q = odd ? r2 : rcv;
 }
 
 // alpha c2r (analysis): sequence t = row pair pidx = p0 + t of one g.
@@ -2341,25 +2365,29 @@ __device__ __forceinline__ void alpha_c2r_body(const AlphaArgs &a, int npt, doub
     int kv[NB][2];
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
-      const int b = threadIdx.x + NT * q, t = b >> (LOGM - 2), jj = b & (Q - 1), pidx = p0 + t;
-      const double2 *rb = a.Tb + ((long long)g * 2 * hi + 2 * pidx) * hi;
+      // rows of one k are adjacent in memory: sequences run along the lanes
+      const int b = threadIdx.x + NT * q, t = b & ((1 << logTw) - 1), jj = b >> logTw, pidx = p0 + t;
+      const double2 *rb = a.Tb + (long long)g * 2 * hi * hi + 2 * pidx * a.tbb;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int k = jj + h * Q;
+        auto at = [=](int i) { return i < hi ? i : i < n ? n - i : 0; };
         kv[q][h] = pidx < hi && k < n ? k : -1;
-        const int kk = k < hi ? k : n - k;
         pk[q][h] = qk[q][h] = make_double2(0.0, 0.0);
         ck[q][h] = make_double2(0.0, 0.0);
-        if (kv[q][h] >= 0) {
-          pk[q][h] = rb[kk];
-          qk[q][h] = rb[hi + kk];
+        if constexpr (LOGM == LOGTS) {
+          load_pair(rb, a.tbb, a.tbm, at(k & ~1), at(k | 1), pk[q][h], qk[q][h]);
+          ck[q][h] = f.chirp[k];
+        } else if (kv[q][h] >= 0) {
+          pk[q][h] = rb[at(k) * a.tbm];
+          qk[q][h] = rb[at(k) * a.tbm + a.tbb];
           ck[q][h] = f.chirp[k];
         }
       }
     }
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
-      const int b = threadIdx.x + NT * q, t = b >> (LOGM - 2), jj = b & (Q - 1);
+      const int b = threadIdx.x + NT * q, t = b & ((1 << logTw) - 1), jj = b >> logTw;
       double2 v[4];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
@@ -2424,28 +2452,31 @@ __device__ __forceinline__ void alpha_c2r_body(const AlphaArgs &a, int npt, doub
 #pragma unroll
   for (int e = 0; e < kTE; ++e) {
     const int s = threadIdx.x + NT * e;
-    const int t = s >> logM, kk = s & (M - 1);
-    if (kk >= n) lds[lpad((kk << logTw) + t)] = make_double2(0.0, 0.0);
+    if ((s >> logTw) >= n) lds[lpad(s)] = make_double2(0.0, 0.0);
   }
   // each Tb element (k < hi) is read once and gives slot k and slot n - k:
   // z_k = p + i q, z_{n-k} = conj(p) + i conj(q) for the packed rows p, q;
   // two rounds of kTE/4 elements per thread keep the loads in flight within
   // the register budget of three waves per SIMD
-  const int logH = logM - 1;  // M/2 >= hi positions per sequence
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
     constexpr int HE = kTE / 4;
     double2 pv[HE], qv[HE], c0[HE], c1[HE];
 #pragma unroll
     for (int e = 0; e < HE; ++e) {
+      // M/2 >= hi positions per sequence, sequences along the lanes
       const int u = threadIdx.x + NT * (e + half * HE);
-      const int t = u >> logH, kk = u & ((1 << logH) - 1), pidx = p0 + t;
+      const int t = u & ((1 << logTw) - 1), kk = u >> logTw, pidx = p0 + t;
+      const double2 *rb = a.Tb + (long long)g * 2 * hi * hi + 2 * pidx * a.tbb;
       pv[e] = qv[e] = make_double2(0.0, 0.0);
       c0[e] = c1[e] = make_double2(1.0, 0.0);
+      if constexpr (LOGM == LOGTS)
+        load_pair(rb, a.tbb, a.tbm, (kk & ~1) < hi ? kk & ~1 : 0, (kk | 1) < hi ? kk | 1 : 0, pv[e], qv[e]);
       if (pidx < hi && kk < hi) {
-        const double2 *rb = a.Tb + ((long long)g * 2 * hi + 2 * pidx) * hi;
-        pv[e] = rb[kk];
-        qv[e] = rb[hi + kk];
+        if constexpr (LOGM != LOGTS) {
+          pv[e] = rb[kk * a.tbm];
+          qv[e] = rb[kk * a.tbm + a.tbb];
+        }
         if (bluestein) {
           c0[e] = f.chirp[kk];
           c1[e] = f.chirp[kk ? n - kk : 0];
@@ -2455,7 +2486,7 @@ __device__ __forceinline__ void alpha_c2r_body(const AlphaArgs &a, int npt, doub
 #pragma unroll
     for (int e = 0; e < HE; ++e) {
       const int u = threadIdx.x + NT * (e + half * HE);
-      const int t = u >> logH, kk = u & ((1 << logH) - 1), pidx = p0 + t;
+      const int t = u & ((1 << logTw) - 1), kk = u >> logTw, pidx = p0 + t;
       if (kk >= hi) continue;
       const double2 p = pv[e], q = qv[e];
       double2 z = kk == 0 ? make_double2(p.x, q.x) : make_double2(p.x - q.y, p.y + q.x);
@@ -2960,14 +2991,12 @@ __global__ __launch_bounds__(NT, 3) void k_alpha_c2r_o2(const AlphaArgs a0, cons
   const int g = tile / npt, p0 = (tile - g * npt) * T;
   // slot k < hi: p_k + i q_k (k = 0: Re p_0 + i Re q_0), slot n - k:
   // conj(p_k) + i conj(q_k), for the packed rows p = 2 pidx, q = 2 pidx + 1
-  for (int idx = threadIdx.x; idx < hi * T; idx += NT) {
-    const int t = idx % T, kk = idx / T, pidx = p0 + t;
-    double2 p = make_double2(0.0, 0.0), q = p;
-    if (pidx < hi) {
-      const double2 *rb = a.Tb + ((long long)g * 2 * hi + 2 * pidx) * hi;
-      p = rb[kk];
-      q = rb[hi + kk];
-    }
+  static_assert(T == 1 && hi % NT == 0 && NT % 2 == 0, "load_pair: one row pair, whole rounds of lane pairs");
+#pragma unroll
+  for (int i = 0; i < hi / NT; ++i) {
+    const int t = 0, kk = threadIdx.x + NT * i;
+    double2 p, q;
+    load_pair(a.Tb + (long long)g * 2 * hi * hi + 2 * p0 * a.tbb, a.tbb, a.tbm, kk & ~1, kk | 1, p, q);
     lds[kk * T + t] = kk == 0 ? make_double2(p.x, q.x) : make_double2(p.x - q.y, p.y + q.x);
     if (kk) lds[(n - kk) * T + t] = make_double2(p.x + q.y, -p.y + q.x);
   }
@@ -3045,23 +3074,34 @@ __global__ __launch_bounds__((1 << LOGM) / 16, MOM && LOGM == 12 ? 2 : 3) void k
   const int g = tile / npt, pidx = tile - g * npt;  // npt = hi
   double2 v[16];
   {
-    const double2 *rb = a.Tb + ((long long)g * 2 * hi + 2 * pidx) * hi;
-    double2 p[8], q[8], c[8];
+    const double2 *rb = a.Tb + (long long)g * 2 * hi * hi + 2 * pidx * a.tbb;
+    // slots k < hi <= M/4 in registers, slot n - k through LDS: reading the
+    // rows a second time from L2 for it costs more
+    double2 p[4], q[4];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const int k = threadIdx.x + NT * r, kk = k < hi ? k : k < n ? n - k : 0;
-      p[r] = rb[kk];
-      q[r] = rb[hi + kk];
-      c[r] = a.f.chirp[k];  // zero for n <= k < M
+    for (int r = 0; r < 4; ++r) {
+      const int k = threadIdx.x + NT * r;
+      load_pair(rb, a.tbb, a.tbm, min(k & ~1, hi - 1), min(k | 1, hi - 1), p[r], q[r]);
     }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int k = threadIdx.x + NT * r;
+      v[r] = k == 0 ? make_double2(p[r].x, q[r].x) : make_double2(p[r].x - q[r].y, p[r].y + q[r].x);
+      if (k >= 1 && k < hi) dyn_lds[hi - 1 - k] = make_double2(p[r].x + q[r].y, -p[r].y + q[r].x);
+    }
+    lds_barrier();
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       const int k = threadIdx.x + NT * r;
-      const double2 z = k == 0  ? make_double2(p[r].x, q[r].x)
-                        : k < hi ? make_double2(p[r].x - q[r].y, p[r].y + q[r].x)
-                                 : make_double2(p[r].x + q[r].y, -p[r].y + q[r].x);
-      v[r] = k < n ? cmulw<+1>(z, c[r]) : make_double2(0.0, 0.0);
+      double2 z = make_double2(0.0, 0.0);
+      if (k < hi) {
+        if (r < 4) z = v[r & 3];
+      } else if (k < n) {
+        z = dyn_lds[k - hi];
+      }
+      v[r] = cmulw<+1>(z, a.f.chirp[k]);  // the chirp table is zero for n <= k < M
     }
+    lds_barrier();
   }
   team16_bluestein<LOGM, +1>(a.f, (double *)dyn_lds, v);
   if constexpr (MOM) {
@@ -3215,19 +3255,19 @@ __device__ __forceinline__ void beta_ana_h2_body(const BetaAnaArgs &a, int nmt, 
   }
   lds_barrier();
   team_fft_core<kTE, NT, -1>(a.f, lds, M, logTw, BL, BL ? a.f.chirp_c : nullptr);
+  // lanes along b, so that the stores of a column are contiguous where tbb = 1
 #pragma unroll
-  for (int e = 0; e < kTE / 2; ++e) {
-    const int s = threadIdx.x + NT * e;
-    const int t = s & (Tw - 1), nn = s >> logTw, m = m0 + t;
-    if (m < hi && (!BL || nn < hi)) {
-      double2 ye = lds[lpad((nn << logTw) + t)], yo = lds[lpad(((L - 1 - nn) << logTw) + t)];
+  for (int e = 0; e < kTE; ++e) {
+    const int s = threadIdx.x + NT * e;  // < Tw M
+    const int t = s >> LOGM, b = s & (M - 1), m = m0 + t;
+    if (m < hi && (!BL || b < L)) {
+      const bool up = b & 1;
+      double2 y = lds[lpad(((up ? L - 1 - (b >> 1) : b >> 1) << logTw) + t)];
       if ((m + N - 1) & 1) {
         const double2 x0 = a.Tg[(long long)g * hi * hi + m];
-        ye = cadd(x0, ye);
-        yo = csub(x0, yo);
+        y = up ? csub(x0, y) : cadd(x0, y);
       }
-      a.Tb[((long long)g * L + 2 * nn) * hi + m] = ye;
-      a.Tb[((long long)g * L + 2 * nn + 1) * hi + m] = yo;
+      a.Tb[(long long)g * L * hi + b * a.tbb + m * a.tbm] = y;
     }
   }
 }
@@ -3379,14 +3419,14 @@ __global__ __launch_bounds__((1 << LOGM) / 16, 3) void k_beta_ana16(const BetaAn
   }
   team16_bluestein<LOGM, -1>(a.f, (double *)dyn_lds, v);
   const double2 x0 = odd ? T[0] : make_double2(0.0, 0.0);
-  double2 *o = a.Tb + (long long)g * L * hi + m;
+  double2 *o = a.Tb + (long long)g * L * hi + m * a.tbm;
 #pragma unroll
   for (int r = 0; r < 8; ++r) {
     const int k = threadIdx.x + NT * r;
     if (k < L) {
       const double2 y = cmulw<-1>(v[r], a.f.chirp[k]);
       const bool up = k >= hi;  // Tb(2n) = [x0 +] v_n, Tb(2n+1) = [x0 -] v_{L-1-n}
-      o[(long long)(up ? 2 * (L - 1 - k) + 1 : 2 * k) * hi] = up && odd ? csub(x0, y) : cadd(x0, y);
+      o[(up ? 2 * (L - 1 - k) + 1 : 2 * k) * a.tbb] = up && odd ? csub(x0, y) : cadd(x0, y);
     }
   }
 }
@@ -4737,6 +4777,16 @@ int launch_syn_nc(int nc, dim3 grid, hipStream_t s, const SynArgs &a) {
 
 bool scale_empty(const Scale &s) { return s.lo + 1 > s.hi - 1; }
 
+// Layout of the analysis's beta output Tb of one g: [m][b], so that the beta
+// kernels, one column m per FFT, store whole cache lines; the alpha kernels
+// read the two adjacent b of a row pair, 32 bytes per m, with the other pairs
+// of a line on the same XCD.  At L = 1024, N = 8 (805 MB in and out) columns
+// stored 16 bytes at a time took 447 us by themselves against 287 us whole,
+// and the 32-byte reads of the alpha stage no more than contiguous ones (227
+// us).  The reference-rounding form's GEMM writes [b][m].
+int tb_stride_b(const Plan *p, int hi) { return p->refround ? hi : 1; }
+int tb_stride_m(const Plan *p, int hi) { return p->refround ? 1 : 2 * hi; }
+
 // Stage arguments of scale j (the launch shape fields are set by the caller).
 BetaAnaArgs make_beta_ana(const Plan *p, int j) {
   const Scale &s = p->sc[j];
@@ -4747,6 +4797,8 @@ BetaAnaArgs make_beta_ana(const Plan *p, int j) {
   b.N = p->N;
   b.Tg = p->d_tg + s.tg_off;
   b.Tb = p->d_tb + s.tb_off;
+  b.tbb = tb_stride_b(p, s.hi);
+  b.tbm = tb_stride_m(p, s.hi);
   b.tw8 = p->d_tw8 + p->tw8_off[j];
   return b;
 }
@@ -4758,6 +4810,8 @@ AlphaArgs make_alpha(const Plan *p, int j, bool synthesis) {
   al.logT = fft_logT(al.f, 4);
   al.hi = s.hi;
   al.Tb = p->d_tb + s.tb_off;
+  al.tbb = tb_stride_b(p, s.hi);
+  al.tbm = tb_stride_m(p, s.hi);
   al.woff = s.wav_off;
   if (synthesis) {
     al.V = p->d_tb + s.tb_off;
@@ -5207,14 +5261,7 @@ int run_analysis(Plan *p, double *d_wav, double2 *d_scoeff, const double2 *d_flm
     // beta
     if (!refb) {
       StageTimer tm(p, 2);
-      BetaAnaArgs b{};
-      b.f = p->ffts[s.fb];
-      b.logT = fft_logT(b.f, 4);
-      b.hi = s.hi;
-      b.N = N;
-      b.Tg = p->d_tg + s.tg_off;
-      b.Tb = p->d_tb + s.tb_off;
-      b.tw8 = p->d_tw8 + p->tw8_off[j];
+      BetaAnaArgs b = make_beta_ana(p, j);
       const WaveShape ws = wave_shape(p, b.f);
       const TeamShape ts = beta_shape(p, b.f, s.hi);
       if (ts.lg >= 0) {
@@ -5237,11 +5284,7 @@ int run_analysis(Plan *p, double *d_wav, double2 *d_scoeff, const double2 *d_flm
     // alpha
     {
       StageTimer tm(p, 3);
-      AlphaArgs al{};
-      al.f = p->ffts[s.fa];
-      al.logT = fft_logT(al.f, 4);
-      al.hi = s.hi;
-      al.Tb = p->d_tb + s.tb_off;
+      AlphaArgs al = make_alpha(p, j, false);
       al.W = wj;
       const WaveShape ws = wave_shape(p, al.f);
       const TeamShape ts = alpha_shape(p, al.f);
