@@ -191,8 +191,10 @@ struct Plan {
   bool syn_mfma = true;       // synthesis contraction on FP64 MFMA
   bool syn_wave = true;       // ... with independent waves (else a V tile staged in LDS)
   int smf_NCp = 0, smf_CW = 0, smf_nch = 0, n_swork = 0;
-  int smf_wcount[3] = {0, 0, 0};  // work items per k-step class (<=2, <=4, <=8)
-  bool smf_side_small = false;     // classes 1, 2 read only scales j >= 2
+  // work lists of the synthesis contraction (0: independent waves, 1: shared
+  // V tile): items per k-step class (<=2, <=4, <=8)
+  int smf_wcount[2][3] = {};
+  bool smf_side_small[2] = {false, false};  // classes 1, 2 read only scales j >= 2
   std::vector<int> smf_lb, smf_ub;
   std::vector<long long> smf_btoff;
   double *d_BT = nullptr;     // per-scale synthesis B tables
@@ -218,7 +220,7 @@ struct Plan {
   bool odd_alpha = true;      // full-band alpha stages of 2hi - 1 = 1023 on the odd-length engine
   bool beta_one = true;       // full-band beta stages with one FFT per column (k_beta_*_h2)
   bool syn_xcd = true;        // synthesis contraction: consecutive work items share an XCD's L2
-  int syn_cw_min = 8;         // synthesis contraction: smallest m' chunk width
+  int syn_cw_min = 4;         // synthesis contraction: smallest m' chunk width
   double2 *d_otw = nullptr;   // its twiddles e^{+2 pi i k/1023} (set when that engine runs)
   // HIP graphs of whole transforms for the device API: one executable graph
   // per (direction, buffers), captured on `cap` at first use and replayed

@@ -1467,6 +1467,11 @@ __global__ __launch_bounds__(256, KSMAX <= 2 ? 3 : KSMAX <= 4 ? 2 : 1) void k_sy
   }
 }
 
+// A wave of 16 l from lw with m-tile m0 and a chunk from m' = bot up.
+__host__ __device__ __forceinline__ bool syn_wave_idle(int lw, int m0, int bot, int L) {
+  return lw >= L || lw + 15 < m0 || lw + 15 < bot;
+}
+
 // Same contraction with every wave independent inside the m' loop: each
 // lane loads its V operand (Vt_j(c, m', m) for its k = c and row m) straight
 // into the MFMA A layout in the register ring, so no V tile is staged in LDS
@@ -1481,21 +1486,25 @@ __global__ __launch_bounds__(256, KSMAX <= 2 ? 3 : KSMAX <= 4 ? 2 : 1) void k_sy
   static_assert(TM == 1, "one 16-row m-tile per wave");
   constexpr int MW = 16 * TM;                        // m per workgroup
   constexpr int DS = 3;                              // register slots: steps in flight
-  __shared__ int s_j[kSynWgSc];
+  __shared__ int s_jw[4][kSynWgSc];
   const int4 wk = a.work[a.work0 + (a.xcd ? xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x)];
   const int l0 = wk.x, m0 = wk.y, ch = wk.z;
   const int L = a.L, NCp = a.NCp;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  // scales active anywhere in [l0, l0 + 63]
+  // scales active anywhere in the wave's own 16 l: a tile of 64 l that spans
+  // more scales costs each wave only its own (two at dilation 2)
+  const int lw = uniform(l0 + 16 * wave);
+  int *s_j = s_jw[wave];
   int nsw = 0;
   for (int j = 0; j < a.nsc; ++j) {
-    if (a.lb[j] <= a.ub[j] && a.lb[j] <= l0 + 63 && a.ub[j] >= l0) {
-      if (threadIdx.x == 0) s_j[nsw] = j;
+    if (a.lb[j] <= a.ub[j] && a.lb[j] <= lw + 15 && a.ub[j] >= lw) {
+      if (lane == 0) s_j[nsw] = j;
       ++nsw;
     }
   }
   const int K = nsw * NCp, KS = K >> 2, kpc = NCp >> 2;
-  const int top = min((ch + 1) * a.CW, L) - 1, bot = ch * a.CW;
+  // the wave's m' <= l ends at lw + 15
+  const int top = min(min((ch + 1) * a.CW, L) - 1, lw + 15), bot = ch * a.CW;
   const int nst = top - bot + 1;  // m' steps, m' = top - i
   const int l = l0 + 16 * wave + (lane & 15);
   const bool lval = l < L;
@@ -1519,6 +1528,12 @@ __global__ __launch_bounds__(256, KSMAX <= 2 ? 3 : KSMAX <= 4 ? 2 : 1) void k_sy
       }
     }
   lds_barrier();  // s_j
+  // nothing of the wave's l reaches this m-tile (m <= l) or chunk (m' <= l):
+  // the assembly never reads its partial sums
+  if (syn_wave_idle(lw, m0, bot, L)) return;
+  // only a chunk that some l of the wave lies in or below starts chains
+  // inside the loop; below the wave's l they start at the checkpoint
+  const bool starts = top >= lw;
   // table form: element off(l) + m'(l+1) + mq + 4r as a byte offset, from
   // m' = top down by l+1 per step (lanes past L use row L-1; offsets that
   // wrap below zero or pass the table read zeros)
@@ -1628,7 +1643,7 @@ __global__ __launch_bounds__(256, KSMAX <= 2 ? 3 : KSMAX <= 4 ? 2 : 1) void k_sy
       const int i = i0 + u;
       if (i >= nst) break;  // uniform
       const int mp = top - i;
-      if (!TAB && mp == l) {
+      if (!TAB && starts && mp == l) {
 #pragma unroll
         for (int t = 0; t < TM; ++t)
 #pragma unroll
@@ -4423,11 +4438,13 @@ int plan_build(Plan *p, int B, int N, int J, double alpha, const double *K, cons
   // checkpoint planes, chunk partials and the work list
   if (p->syn_mfma && NCs > 0) {
     const int NCp = (NCs + 3) & ~3;
-    // m' chunk width ~L/16 (a power of two, at least 8): 16 chunks of work
-    // items at every band limit (small plans get as many workgroups per
-    // l-block as large ones, not one long chain per m-tile)
-    int CW = p->syn_cw_min;
-    while (CW * 16 < L) CW *= 2;
+    // m' chunk width L/16, at least 4: 16 chunks of work items at every band
+    // limit (small plans get as many workgroups per l-block as large ones, and
+    // the tiles of the lowest l, a few workgroups whose steps wait on memory,
+    // stay short).  Synthesis at widths 16, 20, 25, 32, 40 of L = 397: 206, 203,
+    // 200, 205, 213 us; 16, 24, 32, 36 of L = 512: 242, 233, 230, 229 us;
+    // 2, 3, 4, 6, 8 of L = 64: 35, 33, 32, 32, 33 us.
+    const int CW = std::max(p->syn_cw_min, (L + 15) / 16);
     const int nch = (L + CW - 1) / CW;
     const int MW = 16 * kSynTM;
     bool ok = NCp <= 4 * kSynWgSc;
@@ -4437,29 +4454,54 @@ int plan_build(Plan *p, int B, int N, int J, double alpha, const double *K, cons
       ub[j] = p->sc[j].hi - 1;
     }
     // work items (l0, m0, chunk, k-steps), grouped by the k-step class
-    // {<=2, <=4, <=8} of the kernel that runs them
-    std::vector<int4> wcls[3];
-    bool side_small = true;
+    // {<=2, <=4, <=8} of the kernel that runs them: by the most scales that
+    // one of its waves sees (independent waves), and by those of its 64 l
+    // (the kernel with a shared V tile; its list follows the other)
+    std::vector<int4> wcls[2][3];
+    bool side_small[2] = {true, true};
     for (int l0 = ((L - 1) / 64) * 64; l0 >= 0 && ok; l0 -= 64) {
-      int nsw = 0, jmin = Jp1;
-      for (int j = 0; j < Jp1; ++j)
-        if (lb[j] <= ub[j] && lb[j] <= l0 + 63 && ub[j] >= l0) {
-          ++nsw;
-          jmin = std::min(jmin, j);
-        }
+      auto scales = [&](int la, int lz, int *jmin) {
+        int n = 0;
+        for (int j = Jp1 - 1; j >= 0; --j)
+          if (lb[j] <= ub[j] && lb[j] <= lz && ub[j] >= la) {
+            ++n;
+            *jmin = j;
+          }
+        return n;
+      };
+      auto cls_of = [](int ks) { return ks <= 2 ? 0 : ks <= 4 ? 1 : 2; };
+      int jmin = Jp1;
+      const int nsw = scales(l0, l0 + 63, &jmin);
       if (nsw > kSynWgSc || nsw * NCp > 4 * kSynWgSc) ok = false;
-      const int ks = nsw * NCp / 4;
-      const int cls = ks <= 2 ? 0 : ks <= 4 ? 1 : 2;
-      if (cls > 0 && jmin < 2) side_small = false;
-      const int lmax = std::min(l0 + 63, L - 1);
+      const int lmax = std::min(l0 + 63, L - 1), ks = nsw * NCp / 4;
+      if (cls_of(ks) > 0 && jmin < 2) side_small[1] = false;
       for (int c = 0; c * CW <= lmax; ++c)
-        for (int m0 = 0; m0 <= lmax; m0 += MW) wcls[cls].push_back(make_int4(l0, m0, c, ks));
+        for (int m0 = 0; m0 <= lmax; m0 += MW) {
+          wcls[1][cls_of(ks)].push_back(make_int4(l0, m0, c, ks));
+          int kw = 0, jw = Jp1;
+          for (int w = 0; w < 4; ++w) {
+            const int lw = l0 + 16 * w;
+            if (!syn_wave_idle(lw, m0, c * CW, L)) kw = std::max(kw, scales(lw, lw + 15, &jw) * NCp / 4);
+          }
+          if (cls_of(kw) > 0 && jw < 2) side_small[0] = false;
+          wcls[0][cls_of(kw)].push_back(make_int4(l0, m0, c, kw));
+        }
+    }
+    // at most one item per CU: one launch of the largest class, whose
+    // registers cost nothing there
+    if (wcls[0][0].size() + wcls[0][1].size() + wcls[0][2].size() <= 256) {
+      const int top = !wcls[0][2].empty() ? 2 : !wcls[0][1].empty() ? 1 : 0;
+      for (int c = 0; c < top; ++c) {
+        wcls[0][top].insert(wcls[0][top].end(), wcls[0][c].begin(), wcls[0][c].end());
+        wcls[0][c].clear();
+      }
     }
     std::vector<int4> work;
-    for (int c = 0; c < 3; ++c) {
-      p->smf_wcount[c] = (int)wcls[c].size();
-      work.insert(work.end(), wcls[c].begin(), wcls[c].end());
-    }
+    for (int k = 0; k < 2; ++k)
+      for (int c = 0; c < 3; ++c) {
+        p->smf_wcount[k][c] = (int)wcls[k][c].size();
+        work.insert(work.end(), wcls[k][c].begin(), wcls[k][c].end());
+      }
     {
       // the kernel reads Vt, BT and cc through buffer loads with 32-bit offsets
       long long bt = 4;
@@ -4468,7 +4510,7 @@ int plan_build(Plan *p, int B, int N, int J, double alpha, const double *K, cons
       ok = ok && p->tg_doubles * 8 <= kBufMaxBytes && bt * 8 <= kBufMaxBytes && 16LL * L * L <= kBufMaxBytes;
     }
     if (ok) {
-      p->smf_side_small = side_small;
+      for (int k = 0; k < 2; ++k) p->smf_side_small[k] = side_small[k];
       p->smf_NCp = NCp;
       p->smf_CW = CW;
       p->smf_nch = nch;
@@ -5445,8 +5487,9 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
   // j >= 2 when smf_side_small holds: they then run on the helper stream
   // right after those scales' transforms, beside the full-band scales'
   // transforms on the main stream, and the main class needs no fork
-  const bool early = conc && p->syn_mfma && p->smf_side_small && p->smf_wcount[0] > 0 &&
-                     (p->smf_wcount[1] + p->smf_wcount[2]) > 0;
+  const int wk = p->tab_syn || p->syn_wave ? 0 : 1;  // work list of the kernel that runs
+  const int *wcount = p->smf_wcount[wk];
+  const bool early = conc && p->syn_mfma && p->smf_side_small[wk] && wcount[0] > 0 && (wcount[1] + wcount[2]) > 0;
   if (conc) {
     S2DW_HIP_CHECK(hipEventRecord(p->join, p->aux));
     S2DW_HIP_CHECK(hipStreamWaitEvent(st, p->join, 0));
@@ -5485,15 +5528,15 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
       // free on a CU: they are launched first, on the main stream, so that
       // they take their CUs before the main class (on the helper stream)
       // fills the rest
-      const bool side = !early && !p->single_stream && p->smf_wcount[0] > 0 &&
-                        (p->smf_wcount[1] + p->smf_wcount[2]) > 0;
+      const bool side = !early && !p->single_stream && wcount[0] > 0 && (wcount[1] + wcount[2]) > 0;
       if (side) {
         S2DW_HIP_CHECK(hipEventRecord(p->fork, st));
         S2DW_HIP_CHECK(hipStreamWaitEvent(p->aux, p->fork, 0));
       }
-      const int w0[3] = {0, p->smf_wcount[0], p->smf_wcount[0] + p->smf_wcount[1]};
+      const int wb = wk ? p->smf_wcount[0][0] + p->smf_wcount[0][1] + p->smf_wcount[0][2] : 0;
+      const int w0[3] = {wb, wb + wcount[0], wb + wcount[0] + wcount[1]};
       for (int c : {2, 1, 0}) {
-        const int n = p->smf_wcount[c];
+        const int n = wcount[c];
         if (n > 0) {
           const int ksm = 2 << c;
           const size_t lds = 2 * (size_t)ksm * 4 * 16 * TM * sizeof(double2);
