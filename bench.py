@@ -74,8 +74,9 @@ def stage_bytes(hi, lo, N, ncs, grouped=True):
     'small' stages cover scales 2..J; otherwise the FFT stages cover all."""
     def beta_a(h): return N * h * h * 16 + N * 2 * h * h * 16
     def alpha_a(h): return N * 2 * h * h * 16 + N * 2 * h * (2 * h - 1) * 8
-    def alpha_s(h): return N * 2 * h * (2 * h - 1) * 8 + N * 2 * h * h * 16
-    def beta_s(h): return N * 2 * h * h * 16 + ncs * h * h * 16
+    # the gamma-DFT is in the alpha stage: one plane per n-index, not per gamma
+    def alpha_s(h): return N * 2 * h * (2 * h - 1) * 8 + ncs * 2 * h * h * 16
+    def beta_s(h): return ncs * 2 * h * h * 16 + ncs * h * h * 16
     sc = [j for j, (h, l_) in enumerate(zip(hi, lo)) if l_ + 1 <= h - 1]
     big = [hi[j] for j in sc if j < 2 or not grouped]
     small = [hi[j] for j in sc if j >= 2 and grouped]
@@ -335,10 +336,10 @@ def bench_serve(args, precision=0):
 
 
 # stage name -> kernel whose launches dominate it
-STAGE_KERNEL = {"ana_contract": "k_ana_contract_mfma_w", "syn_contract": "k_syn_contract_mfma",
+STAGE_KERNEL = {"ana_contract": "k_ana_contract_par", "syn_contract": "k_syn_contract_mfma",
                 "ana_beta_fft": "k_beta_ana_h2", "ana_alpha_c2r": "k_alpha_c2r_o2",
-                "syn_alpha_r2c": "k_alpha_r2c_o2", "syn_beta_fft": "k_beta_syn_h2",
-                "ana_small_ffts": "k_alpha_c2r_g", "syn_small_ffts": "k_alpha_r2c_g"}
+                "syn_alpha_r2c": "k_alpha_syn_o2", "syn_beta_fft": "k_beta_syn_h2",
+                "ana_small_ffts": "k_alpha_c2r_g", "syn_small_ffts": "k_alpha_syn_g"}
 
 
 def load_traffic(stage):

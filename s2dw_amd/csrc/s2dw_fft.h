@@ -843,10 +843,17 @@ __device__ __forceinline__ void exchange16(double *buf, double2 (&v)[16], Wr wr,
 // k >= n; k >= M/2 is zero).  Out: v[r] = convolution output k = threadIdx.x
 // + NT r, to be multiplied by chirp_k^{DIR} (k < n <= M/2, so r < 8).  buf:
 // lpad16(M) doubles, free again after a barrier.
-template <int LOGM, int DIR>
+//
+// GRP: the workgroup holds several sequences of NT = M/16 threads, each with
+// its own buf; threadIdx.x stands for its remainder mod NT above.
+template <int LOGM, int DIR, bool GRP = false>
 __device__ __forceinline__ void team16_bluestein(const FftSpec &s, double *buf, double2 (&v)[16]) {
   constexpr int M = 1 << LOGM, NT = M / 16, R3 = M / 256, NC = 16 / R3;
-  static_assert(R3 == 16 || R3 == 8, "M = 4096 or 2048");
+  static_assert(R3 >= 2 && R3 <= 16, "M = 512 .. 4096");
+  auto stage_tid = [] {
+    const int t = s2dw::stage_tid();
+    return GRP ? t & (NT - 1) : t;
+  };
   const double2 *__restrict__ tw = s.tw;
   const double2 *__restrict__ F = DIR > 0 ? s.filt_b : s.filt_f;
   // forward, Ns = 1
@@ -869,9 +876,9 @@ __device__ __forceinline__ void team16_bluestein(const FftSpec &s, double *buf, 
     for (int q = 0; q < NC; ++q) {
       const int jj = tid + NT * q;
       w1[q] = tw[jj];
-      w2[q] = tw[2 * jj];
-      w4[q] = tw[4 * jj];
-      w8[q] = R3 == 16 ? tw[8 * jj] : w4[q];
+      w2[q] = R3 > 2 ? tw[2 * jj] : w1[q];
+      w4[q] = R3 > 4 ? tw[4 * jj] : w1[q];
+      w8[q] = R3 > 8 ? tw[8 * jj] : w1[q];
     }
     const int wb = (tid - jm) * 17 + jm, rb = lpad16(tid);
     exchange16(buf, v, [=](int r) { return wb + 17 * r; },

@@ -2553,7 +2553,8 @@ __device__ __forceinline__ void alpha_c2r_body_m(const AlphaArgs &a, int npt, do
   alpha_c2r_body<LOGM, BL, true>(a, npt, lds, bid, nb);
 }
 
-// alpha r2c (synthesis): sequence t = row pair pidx = p0 + t of one g.
+// alpha r2c (synthesis) of packed real rows, for scales whose beta stage does
+// the gamma-DFT: sequence t = row pair pidx = p0 + t of one g.
 template <int LOGM, int BL, int NT = kTN>
 __device__ __forceinline__ void alpha_r2c_body(const AlphaArgs &a, int npt, double2 *lds, int bid, int nb) {
   constexpr int LOGTS = clog2(NT * kTE);  // log2 of the workgroup's slots
@@ -2563,43 +2564,6 @@ __device__ __forceinline__ void alpha_r2c_body(const AlphaArgs &a, int npt, doub
   const int logTw = LOGM > 0 ? LOGTS - LOGM : a.logT;
   const int tile = xcd_tile(bid, nb);
   const int g = tile / npt, p0 = (tile - g * npt) << logTw;
-  if constexpr (LOGM > 0 && LOGM % 3 == 2 && BL == 1) {
-    // Bluestein's radix-4 first stage from the loaded rows: slots k < n hold
-    // (w0_k + i w1_k) conj(chirp_k), slots k >= n are zero and n <= M/2, so
-    // butterfly jj (slots jj + r M/4) has non-zero inputs for r < 2 only.
-    constexpr int Q = 1 << (LOGM - 2), NB = kTE / 4;
-    double x0[NB][2], x1[NB][2];
-    double2 c[NB][2];
-#pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const int b = threadIdx.x + NT * q, t = b >> (LOGM - 2), jj = b & (Q - 1), pidx = p0 + t;
-      const double *w0 = a.W + ((long long)g * 2 * hi + 2 * pidx) * n;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int k = jj + h * Q;
-        x0[q][h] = x1[q][h] = 0.0;
-        c[q][h] = make_double2(0.0, 0.0);
-        if (pidx < hi && k < n) {
-          x0[q][h] = w0[k];
-          x1[q][h] = w0[n + k];
-          c[q][h] = f.chirp[k];
-        }
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < NB; ++q) {
-      const int b = threadIdx.x + NT * q, t = b >> (LOGM - 2), jj = b & (Q - 1);
-      double2 v[4];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) v[h] = cmulw<-1>(make_double2(x0[q][h], x1[q][h]), c[q][h]);
-      v[2] = v[3] = make_double2(0.0, 0.0);
-      dft_pow2<4, -1>(v);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) lds[lpad(((4 * jj + r) << logTw) + t)] = v[r];
-    }
-    lds_barrier();
-    team_fft_core<kTE, NT, -1, true>(f, lds, M, logTw, true, f.chirp_c);
-  } else {
   {
     double x0[kTE], x1[kTE];
     double2 c[kTE];
@@ -2629,7 +2593,6 @@ __device__ __forceinline__ void alpha_r2c_body(const AlphaArgs &a, int npt, doub
   // Bluestein: the final chirp multiply (by conj(chirp) for this direction)
   // is folded into the last stage through a conjugated copy
   team_fft_core<kTE, NT, -1>(f, lds, M, logTw, bluestein, bluestein ? f.chirp_c : nullptr);
-  }
   const double h = 0.5 * a.scale;
   const int logH = logM - 1;  // outputs k < hi <= M/2: slots (t, k) with k < M/2
 #pragma unroll
@@ -3078,15 +3041,19 @@ __global__ __launch_bounds__(NT, 3) void k_alpha_syn_o2(const AlphaArgs a0, cons
 // leave from the last stage's; the slots carry only what another thread needs
 // (the mirrored halves of the packed rows and of the beta columns).
 // ---------------------------------------------------------------------------
-template <int LOGM, bool MOM>
-__global__ __launch_bounds__((1 << LOGM) / 16, MOM && LOGM == 12 ? 2 : 3) void k_alpha_c2r16(const AlphaArgs a0, const AlphaArgs a1, int npt,
-                                                                    int half) {
+// SEQ = 1: the workgroup is one sequence; SEQ > 1 (grouped launches): SEQ
+// sequences of NT threads, row pairs p0 + i of one g.
+template <int LOGM, bool MOM, int SEQ>
+__device__ __forceinline__ void alpha_c2r16_body(const AlphaArgs &a, int npt, double2 *lds, int bid, int nb) {
   constexpr int NT = (1 << LOGM) / 16;
-  extern __shared__ double2 dyn_lds[];
-  const bool second = (int)blockIdx.x >= half;
-  const AlphaArgs &a = second ? a1 : a0;
-  const int hi = a.hi, n = 2 * hi - 1, tile = xcd_tile(blockIdx.x - (second ? half : 0), half);
-  const int g = tile / npt, pidx = tile - g * npt;  // npt = hi
+  static_assert(!MOM || SEQ == 1, "one record per workgroup");
+  const int tid = SEQ > 1 ? threadIdx.x & (NT - 1) : threadIdx.x, sub = SEQ > 1 ? threadIdx.x / NT : 0;
+  const int hi = a.hi, n = 2 * hi - 1, tile = xcd_tile(bid, nb);
+  const int g = tile / npt, pidx0 = (tile - g * npt) * SEQ + sub;
+  const bool on = SEQ == 1 || pidx0 < hi;
+  const int pidx = on ? pidx0 : hi - 1;
+  double *buf = (double *)lds + sub * lpad16(1 << LOGM);
+  double2 *mir = (double2 *)buf;
   double2 v[16];
   {
     const double2 *rb = a.Tb + (long long)g * 2 * hi * hi + 2 * pidx * a.tbb;
@@ -3095,35 +3062,35 @@ __global__ __launch_bounds__((1 << LOGM) / 16, MOM && LOGM == 12 ? 2 : 3) void k
     double2 p[4], q[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int k = threadIdx.x + NT * r;
+      const int k = tid + NT * r;
       load_pair(rb, a.tbb, a.tbm, min(k & ~1, hi - 1), min(k | 1, hi - 1), p[r], q[r]);
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int k = threadIdx.x + NT * r;
+      const int k = tid + NT * r;
       v[r] = k == 0 ? make_double2(p[r].x, q[r].x) : make_double2(p[r].x - q[r].y, p[r].y + q[r].x);
-      if (k >= 1 && k < hi) dyn_lds[hi - 1 - k] = make_double2(p[r].x + q[r].y, -p[r].y + q[r].x);
+      if (k >= 1 && k < hi) mir[hi - 1 - k] = make_double2(p[r].x + q[r].y, -p[r].y + q[r].x);
     }
     lds_barrier();
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      const int k = threadIdx.x + NT * r;
+      const int k = tid + NT * r;
       double2 z = make_double2(0.0, 0.0);
       if (k < hi) {
         if (r < 4) z = v[r & 3];
       } else if (k < n) {
-        z = dyn_lds[k - hi];
+        z = mir[k - hi];
       }
       v[r] = cmulw<+1>(z, a.f.chirp[k]);  // the chirp table is zero for n <= k < M
     }
     lds_barrier();
   }
-  team16_bluestein<LOGM, +1>(a.f, (double *)dyn_lds, v);
+  team16_bluestein<LOGM, +1, (SEQ > 1)>(a.f, buf, v);
   if constexpr (MOM) {
     double x[16], wt[16];
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      const int k = threadIdx.x + NT * r;
+      const int k = tid + NT * r;
       const double2 z = cmulw<+1>(v[r], a.f.chirp[k]);
       x[2 * r] = z.x;
       x[2 * r + 1] = z.y;
@@ -3135,13 +3102,21 @@ __global__ __launch_bounds__((1 << LOGM) / 16, MOM && LOGM == 12 ? 2 : 3) void k
   double *w0 = a.W + ((long long)g * 2 * hi + 2 * pidx) * n;
 #pragma unroll
   for (int r = 0; r < 8; ++r) {
-    const int k = threadIdx.x + NT * r;
-    if (k < n) {
+    const int k = tid + NT * r;
+    if (on && k < n) {
       const double2 z = cmulw<+1>(v[r], a.f.chirp[k]);
       w0[k] = z.x;
       w0[n + k] = z.y;
     }
   }
+}
+
+template <int LOGM, bool MOM>
+__global__ __launch_bounds__((1 << LOGM) / 16, MOM && LOGM == 12 ? 2 : 3) void k_alpha_c2r16(const AlphaArgs a0, const AlphaArgs a1, int npt,
+                                                                    int half) {
+  extern __shared__ double2 dyn_lds[];
+  const bool second = (int)blockIdx.x >= half;
+  alpha_c2r16_body<LOGM, MOM, 1>(second ? a1 : a0, npt, dyn_lds, blockIdx.x - (second ? half : 0), half);
 }
 
 template <int LOGM>
@@ -3549,6 +3524,13 @@ __device__ __forceinline__ int seg_of(const SegTab &t, int b) {
   case 2 * (LM) + (B):             \
     BODY<LM, B>(__VA_ARGS__);      \
     break;
+// three-stage engine in a grouped launch: 4096 >> log2(M) sequences per
+// workgroup, selector kSel16 + log2(M)
+constexpr int kSel16 = 200, kLds16g = (lpad16(4096) + 1) / 2;
+#define S2DW_SEL16(LM, ...)                        \
+  case kSel16 + (LM):                              \
+    __VA_ARGS__;                                   \
+    break;
 // one-FFT-per-column beta bodies: selector kSelH2 + 2 log2(M) + bluestein
 constexpr int kSelH2 = 100;
 #define S2DW_SEL_H2(BODY, LM, B, ...)     \
@@ -3584,7 +3566,7 @@ __global__ __launch_bounds__(kTN, 3) void k_beta_ana_g(const SegTab t, const Bet
 
 __global__ __launch_bounds__(kTN, 3) void k_alpha_c2r_g(const SegTab t, const AlphaArgs *__restrict__ args,
                                                          double *wbase) {
-  __shared__ double2 lds[lpad_size(kTS)];
+  __shared__ double2 lds[kLds16g];
   const int s = seg_of(t, blockIdx.x), bid = blockIdx.x - t.first[s], nb = t.first[s + 1] - t.first[s];
   AlphaArgs a = args[s];
   a.W = wbase + a.woff;
@@ -3594,8 +3576,8 @@ __global__ __launch_bounds__(kTN, 3) void k_alpha_c2r_g(const SegTab t, const Al
     S2DW_SEL(alpha_c2r_body, 7, 1, a, t.par[s], lds, bid, nb)
     S2DW_SEL(alpha_c2r_body, 8, 1, a, t.par[s], lds, bid, nb)
     S2DW_SEL(alpha_c2r_body, 9, 1, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(alpha_c2r_body, 10, 1, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(alpha_c2r_body, 11, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL16(10, alpha_c2r16_body<10, false, (4096 >> 10)>(a, t.par[s], lds, bid, nb))
+    S2DW_SEL16(11, alpha_c2r16_body<11, false, (4096 >> 11)>(a, t.par[s], lds, bid, nb))
     default: alpha_c2r_body<0, -1>(a, t.par[s], lds, bid, nb); break;
   }
 }
@@ -3647,6 +3629,7 @@ __global__ __launch_bounds__(kTN, 3) void k_beta_syn_g(const SegTab t, const Bet
   }
 }
 #undef S2DW_SEL
+#undef S2DW_SEL16
 #undef S2DW_SEL_H2
 #undef S2DW_SEL_H2_ALL
 
@@ -4914,7 +4897,7 @@ int beta_sel(const TeamShape &t) { return t.h2 ? kSelH2 + 2 * t.lg + t.bl : 0; }
 // tables go in the kernel arguments, the stage arguments in device tables.
 struct Group {
   bool ana = false, syn = false;
-  SegTab ba{}, ac{}, ar{}, bs{};
+  SegTab ba{}, ac{}, am{}, ar{}, bs{};  // am: alpha c2r reducing to moments
   BetaAnaArgs *d_ba = nullptr;
   AlphaArgs *d_ac = nullptr, *d_ar = nullptr;
   BetaSynArgs *d_bs = nullptr;
@@ -4969,7 +4952,17 @@ int build_group(Plan *p, GroupState *gs, int gi, int j0, int j1) {
     };
     add(G.ba, nmt * N, beta_sel(tb), nmt);
     add(G.bs, nmt * nn, beta_sel(tb), nmt);
-    add(G.ac, npt * N, alpha_sel(ta), npt);
+    // analysis, work lengths 1024 and 2048: the three-stage engine from 128
+    // workgroups (half a workgroup per CU) on; it holds twice the sequences per
+    // workgroup.  L = 512, N = 8: 254 -> 244 us per analysis, L = 219, N = 7:
+    // 116 -> 111; L = 201, N = 1 (51 workgroups) 53.6 -> 56.0.  In the synthesis
+    // launch, whose gather needs the registers, it spills and small plans lose
+    // 5%.
+    const int np16 = (s.hi + (4096 >> ta.lg) - 1) / (4096 >> ta.lg);
+    const bool e16 = ta.bl && ta.lg >= 10 && np16 * N >= 128;
+    if (e16) add(G.ac, np16 * N, kSel16 + ta.lg, np16);
+    else add(G.ac, npt * N, alpha_sel(ta), npt);
+    add(G.am, npt * N, alpha_sel(ta), npt);
     add(G.ar, syn_blocks(p, s.hi, ta.per), alpha_sel(ta), 0);
     taken.push_back(j);
     ba.push_back(b);
@@ -5244,7 +5237,7 @@ int run_analysis(Plan *p, double *d_wav, double2 *d_scoeff, const double2 *d_flm
     }
     StageTimer tm(p, 9);
     if (d_mom)
-      hipLaunchKernelGGL(k_alpha_c2r_gm, dim3(G.ac.first[G.ac.nseg]), dim3(kTN), 0, sg, G.ac, G.d_ac, p->d_momf);
+      hipLaunchKernelGGL(k_alpha_c2r_gm, dim3(G.am.first[G.am.nseg]), dim3(kTN), 0, sg, G.am, G.d_ac, p->d_momf);
     else
       hipLaunchKernelGGL(k_alpha_c2r_g, dim3(G.ac.first[G.ac.nseg]), dim3(kTN), 0, sg, G.ac, G.d_ac, d_wav);
     S2DW_HIP_CHECK(hipGetLastError());
