@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -16,6 +17,7 @@
 #include <list>
 #include <memory>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 #include "../../include/s2dw_hip.h"
@@ -76,35 +78,63 @@ std::list<std::unique_ptr<HostEntry>> g_cache;  // most recent first
 constexpr size_t kCacheMax = 4;
 
 // Copies between the caller's (pageable) arrays and the device.  Copies of
-// kStageMin and more go through a ring of pinned slots: the DMA of a slot
-// overlaps the host copies of the others, and a host copy is split over
+// kStageMin and more go through a ring of slots in pinned memory: the DMA of a
+// slot overlaps the host copies of the others, and host copies are split over
 // threads.  The scales of a transform, adjacent on the device and separate
-// arrays on the host, are one copy.  At L = 256, N = 5 (24 MB in nine scales)
-// the analysis call into warm arrays takes 940 us and the synthesis 807 us,
-// against 1160 and 884 us with one 32 MB buffer per scale of 10 MB (its DMA
-// and host copy one after the other) and the runtime's pageable copies for
-// the others; 2 MB slots measured the same.  A slot is allocated when first
-// used and kept until the process ends; g_mu guards them.
-constexpr size_t kSlotBytes = 4u << 20, kStageMin = 1u << 20;
-constexpr int kSlots = 16;
+// arrays on the host, are one copy.  The ring grows up to kRingMax with the
+// copies it has served and is kept until the process ends; g_mu guards it.
+constexpr size_t kRingMax = 64u << 20, kSlotMin = 4u << 20, kStageMin = 1u << 20;
+constexpr int kSlots = kRingMax / kSlotMin;
 struct StageSlot {
-  void *buf = nullptr;
   hipEvent_t ev = nullptr;
   bool rec = false;  // the event has been recorded
 };
-StageSlot g_slot[kSlots];
+struct StageRing {
+  char *buf = nullptr;
+  size_t bytes = 0, slot = 0;  // slot: size of the slots of the last copy
+  StageSlot s[kSlots];
+  int n() const { return (int)(bytes / slot); }
+  StageSlot &at(size_t k) { return s[k % n()]; }
+  char *mem(size_t k) const { return buf + (k % n()) * slot; }
+};
+StageRing g_ring;
 
-// The slot, its previous transfer (on whatever stream) finished.
-int slot_ready(StageSlot &s) {
-  if (!s.buf) S2DW_HIP_CHECK(hipHostMalloc(&s.buf, kSlotBytes, hipHostMallocDefault));
-  if (!s.ev) S2DW_HIP_CHECK(hipEventCreateWithFlags(&s.ev, hipEventDisableTiming));
+// The slot's previous transfer, on whatever stream, has finished.
+int slot_wait(const StageSlot &s) {
   if (s.rec) S2DW_HIP_CHECK(hipEventSynchronize(s.ev));
   return kErrNone;
 }
 
 int slot_record(StageSlot &s, hipStream_t st) {
+  if (!s.ev) S2DW_HIP_CHECK(hipEventCreateWithFlags(&s.ev, hipEventDisableTiming));
   S2DW_HIP_CHECK(hipEventRecord(s.ev, st));
   s.rec = true;
+  return kErrNone;
+}
+
+// The ring for a copy of n bytes.  A transfer costs about 16 us beyond its
+// bytes, and the first or last slot's host copy overlaps with nothing, so the
+// slots grow with the copy.  L = 512, N = 8, static arrays (537 MB), analysis
+// into touched arrays and synthesis: slots of 4 MB 16.0 and 15.5 ms, 16 MB 14.2
+// and 13.5, 32 MB 14.0 and 13.3; dynamic arrays (157 MB) 4.67 and 4.14 ms with
+// 4 MB, 4.27 and 3.69 with 16 MB; L = 256, N = 5 (24 MB) 0.94 and 0.79 with
+// 4 MB, 0.92 and 0.75 with 8 MB.
+int ring_ready(size_t n) {
+  const size_t slot = n <= 4 * kSlotMin ? kSlotMin : n <= kRingMax ? 2 * kSlotMin : n <= 4 * kRingMax ? 4 * kSlotMin : 8 * kSlotMin;
+  size_t want = kSlotMin;
+  while (want < n && want < kRingMax) want *= 2;
+  if (g_ring.slot == slot && g_ring.bytes >= want) return kErrNone;
+  for (StageSlot &s : g_ring.s)
+    if (int e = slot_wait(s)) return e;
+  g_ring.slot = slot;
+  if (g_ring.bytes >= want) return kErrNone;
+  if (g_ring.buf) (void)hipHostFree(g_ring.buf);
+  g_ring.buf = nullptr;
+  g_ring.bytes = 0;
+  void *q = nullptr;
+  S2DW_HIP_CHECK(hipHostMalloc(&q, want, hipHostMallocDefault));
+  g_ring.buf = static_cast<char *>(q);
+  g_ring.bytes = want;
   return kErrNone;
 }
 
@@ -120,32 +150,41 @@ size_t runs_bytes(const std::vector<HostRun> &runs) {
   return t;
 }
 
-// Bytes [o, o + len) of the runs to or from buf, split over threads.
-void runs_copy(const std::vector<HostRun> &runs, size_t o, size_t len, void *buf, bool to_host) {
-  constexpr size_t kPiece = 256u << 10;
-  const long long np = (long long)((len + kPiece - 1) / kPiece);
-#pragma omp parallel for schedule(static) if (np > 2)
-  for (long long i = 0; i < np; ++i) {
-    size_t a = (size_t)i * kPiece, left = std::min(kPiece, len - a), skip = o + a;
-    for (const HostRun &r : runs) {
-      if (skip >= r.n) {
-        skip -= r.n;
-        continue;
-      }
-      const size_t m = std::min(left, r.n - skip);
-      char *h = static_cast<char *>(r.host) + skip, *b = static_cast<char *>(buf) + a;
-      if (to_host) std::memcpy(h, b, m);
-      else std::memcpy(b, h, m);
-      a += m;
-      left -= m;
-      skip = 0;
-      if (!left) break;
+// Bytes [o, o + len) of the runs to or from b.
+void runs_copy(const std::vector<HostRun> &runs, size_t o, size_t len, char *b, bool to_host) {
+  for (const HostRun &r : runs) {
+    if (o >= r.n) {
+      o -= r.n;
+      continue;
     }
+    const size_t m = std::min(len, r.n - o);
+    char *h = static_cast<char *>(r.host) + o;
+    if (to_host) std::memcpy(h, b, m);
+    else std::memcpy(b, h, m);
+    b += m;
+    len -= m;
+    o = 0;
+    if (!len) break;
   }
+}
+
+// Size of the pieces that threads copy, for len bytes: 16 pieces, between
+// 256 KB and 1 MB.
+size_t piece_of(size_t len) {
+  size_t q = 256u << 10;
+  while (q * 16 < len && q < (1u << 20)) q *= 2;
+  return q;
 }
 
 // Device to host, in stream order after the work already on st; large
 // copies have completed on return, small ones at the next synchronisation.
+// One parallel region copies half a ring (the whole of it where it holds the
+// copy): arrays that the caller has not touched yet take page faults of 2 MB,
+// which serialise the threads that share a page, so the threads of a region
+// are spread over more than one slot (new arrays at L = 512, N = 8: one region
+// per 4 MB in pieces of 256 KB 22.8 ms static and 7.7 ms dynamic, this 14.8 and
+// 4.9).  They take the pieces in order; the one with a slot's first piece waits
+// for the slot's transfer, the others for it.
 int copy_d2h(const std::vector<HostRun> &runs, const void *src, hipStream_t st) {
   const size_t n = runs_bytes(runs);
   const char *d = static_cast<const char *>(src);
@@ -156,19 +195,35 @@ int copy_d2h(const std::vector<HostRun> &runs, const void *src, hipStream_t st) 
     }
     return kErrNone;
   }
-  const size_t nch = (n + kSlotBytes - 1) / kSlotBytes;
+  if (int e = ring_ready(n)) return e;
+  const size_t slot = g_ring.slot, nch = (n + slot - 1) / slot, nring = (size_t)g_ring.n();
+  const size_t group = nch <= nring ? nch : nring / 2, piece = piece_of(group * slot), per = slot / piece;
   size_t issued = 0;
-  for (size_t k = 0; k < nch; ++k) {
-    for (; issued < nch && issued < k + kSlots; ++issued) {
-      StageSlot &s = g_slot[issued % kSlots];
-      if (int e = slot_ready(s)) return e;
-      const size_t o = issued * kSlotBytes;
-      S2DW_HIP_CHECK(hipMemcpyAsync(s.buf, d + o, std::min(kSlotBytes, n - o), hipMemcpyDeviceToHost, st));
+  for (size_t k0 = 0; k0 < nch; k0 += group) {
+    for (; issued < nch && issued < k0 + nring; ++issued) {
+      StageSlot &s = g_ring.at(issued);
+      const size_t o = issued * slot;
+      if (int e = slot_wait(s)) return e;
+      S2DW_HIP_CHECK(hipMemcpyAsync(g_ring.mem(issued), d + o, std::min(slot, n - o), hipMemcpyDeviceToHost, st));
       if (int e = slot_record(s, st)) return e;
     }
-    StageSlot &s = g_slot[k % kSlots];
-    S2DW_HIP_CHECK(hipEventSynchronize(s.ev));
-    runs_copy(runs, k * kSlotBytes, std::min(kSlotBytes, n - k * kSlotBytes), s.buf, true);
+    const size_t o0 = k0 * slot, o1 = std::min(n, (k0 + group) * slot);
+    const long long np = (long long)((o1 - o0 + piece - 1) / piece);
+    std::atomic<int> ready[kSlots], err{(int)hipSuccess};
+    for (auto &r : ready) r.store(0);
+#pragma omp parallel for schedule(dynamic, 1) if (np > 1)
+    for (long long i = 0; i < np; ++i) {
+      const size_t q = (size_t)i / per, p = (size_t)i % per, o = o0 + (size_t)i * piece;
+      if (p == 0) {
+        const hipError_t e = hipEventSynchronize(g_ring.at(k0 + q).ev);
+        if (e != hipSuccess) err.store((int)e);
+        ready[q].store(1, std::memory_order_release);
+      } else {
+        while (!ready[q].load(std::memory_order_acquire)) std::this_thread::yield();
+      }
+      runs_copy(runs, o, std::min(piece, o1 - o), g_ring.mem(k0 + q) + p * piece, true);
+    }
+    S2DW_HIP_CHECK((hipError_t)err.load());
   }
   return kErrNone;
 }
@@ -185,13 +240,20 @@ int copy_h2d(void *dst, const std::vector<HostRun> &runs, hipStream_t st) {
     }
     return kErrNone;
   }
-  const size_t nch = (n + kSlotBytes - 1) / kSlotBytes;
+  if (int e = ring_ready(n)) return e;
+  const size_t slot = g_ring.slot, nch = (n + slot - 1) / slot, piece = piece_of(slot);
   for (size_t k = 0; k < nch; ++k) {
-    StageSlot &s = g_slot[k % kSlots];
-    if (int e = slot_ready(s)) return e;
-    const size_t o = k * kSlotBytes, len = std::min(kSlotBytes, n - o);
-    runs_copy(runs, o, len, s.buf, false);
-    S2DW_HIP_CHECK(hipMemcpyAsync(d + o, s.buf, len, hipMemcpyHostToDevice, st));
+    StageSlot &s = g_ring.at(k);
+    if (int e = slot_wait(s)) return e;
+    const size_t o = k * slot, len = std::min(slot, n - o);
+    char *b = g_ring.mem(k);
+    const long long np = (long long)((len + piece - 1) / piece);
+#pragma omp parallel for schedule(static) if (np > 2)
+    for (long long i = 0; i < np; ++i) {
+      const size_t a = (size_t)i * piece;
+      runs_copy(runs, o + a, std::min(piece, len - a), b + a, false);
+    }
+    S2DW_HIP_CHECK(hipMemcpyAsync(d + o, b, len, hipMemcpyHostToDevice, st));
     if (int e = slot_record(s, st)) return e;
   }
   return kErrNone;
