@@ -3576,6 +3576,7 @@ __global__ __launch_bounds__(kTN, 3) void k_alpha_c2r_g(const SegTab t, const Al
     S2DW_SEL(alpha_c2r_body, 7, 1, a, t.par[s], lds, bid, nb)
     S2DW_SEL(alpha_c2r_body, 8, 1, a, t.par[s], lds, bid, nb)
     S2DW_SEL(alpha_c2r_body, 9, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_c2r_body, 10, 1, a, t.par[s], lds, bid, nb)
     S2DW_SEL16(10, alpha_c2r16_body<10, false, (4096 >> 10)>(a, t.par[s], lds, bid, nb))
     S2DW_SEL16(11, alpha_c2r16_body<11, false, (4096 >> 11)>(a, t.par[s], lds, bid, nb))
     default: alpha_c2r_body<0, -1>(a, t.par[s], lds, bid, nb); break;
@@ -4885,7 +4886,8 @@ BetaSynArgs make_beta_syn(const Plan *p, int j) {
 }
 
 // Body selector of a grouped alpha launch: 2 log2(M) + bluestein for the
-// specialised work lengths (Bluestein, log2 M in [5, 11]), else 0 (generic).
+// specialised work lengths (Bluestein, log2 M in [5, 11]; k_alpha_c2r_g has no
+// 11, which always runs on its three-stage engine), else 0 (generic).
 int alpha_sel(const TeamShape &t) { return t.bl && t.lg >= 5 && t.lg <= kLogTS ? 2 * t.lg + 1 : 0; }
 // ... of a grouped beta launch
 int beta_sel(const TeamShape &t) { return t.h2 ? kSelH2 + 2 * t.lg + t.bl : 0; }
@@ -4926,6 +4928,13 @@ int build_group(Plan *p, GroupState *gs, int gi, int j0, int j1) {
   std::vector<int> taken;
   bool ok = j1 - j0 >= 2 || (gi == 1 && j1 > j0);
   const bool syn_ok = p->gamma_first;
+  // workgroups that the three-stage engine would take of the analysis alpha launch
+  auto wg16_of = [&](const Scale &s, const TeamShape &t) { return (s.hi + (4096 >> t.lg) - 1) / (4096 >> t.lg) * N; };
+  int wg16 = 0;
+  for (int j = j0; j < j1; ++j) {
+    const TeamShape t = scale_empty(p->sc[j]) ? TeamShape{} : alpha_shape(p, p->ffts[p->sc[j].fa]);
+    if (t.bl && (t.lg == 10 || t.lg == 11)) wg16 += wg16_of(p->sc[j], t);
+  }
   for (int j = j0; j < j1 && ok; ++j) {
     const Scale &s = p->sc[j];
     if (scale_empty(s)) {
@@ -4952,14 +4961,15 @@ int build_group(Plan *p, GroupState *gs, int gi, int j0, int j1) {
     };
     add(G.ba, nmt * N, beta_sel(tb), nmt);
     add(G.bs, nmt * nn, beta_sel(tb), nmt);
-    // analysis, work lengths 1024 and 2048: the three-stage engine from 128
-    // workgroups (half a workgroup per CU) on; it holds twice the sequences per
-    // workgroup.  L = 512, N = 8: 254 -> 244 us per analysis, L = 219, N = 7:
-    // 116 -> 111; L = 201, N = 1 (51 workgroups) 53.6 -> 56.0.  In the synthesis
+    // analysis, work length 2048, and 1024 where the launch has a workgroup per
+    // CU of these: the three-stage engine; it holds twice the sequences per
+    // workgroup.  This launch, on it and on the radix-8 body, us: L = 256, N = 2
+    // (256 workgroups) 28.7 and 30.0, N = 4 (512) 38.2 and 41.7; L = 512, N = 2
+    // (128) 27.2 and 25.9, L = 201, N = 1 (102) 28.1 and 25.2.  In the synthesis
     // launch, whose gather needs the registers, it spills and small plans lose
     // 5%.
-    const int np16 = (s.hi + (4096 >> ta.lg) - 1) / (4096 >> ta.lg);
-    const bool e16 = ta.bl && ta.lg >= 10 && np16 * N >= 128;
+    const bool e16 = ta.bl && (ta.lg == 11 || (ta.lg == 10 && wg16 >= 256));
+    const int np16 = e16 ? wg16_of(s, ta) / N : 0;
     if (e16) add(G.ac, np16 * N, kSel16 + ta.lg, np16);
     else add(G.ac, npt * N, alpha_sel(ta), npt);
     add(G.am, npt * N, alpha_sel(ta), npt);
