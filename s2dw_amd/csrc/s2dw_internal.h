@@ -176,7 +176,6 @@ struct Plan {
   double2 *eg = nullptr;      // synthesis gamma table [n-index][g]
   std::vector<int> nlist;     // synthesis n values (n >= 0, N+n odd)
   int z0 = -1;                // index of n = 0 in nlist, -1: none
-  bool gamma_first = false;   // synthesis: gamma-DFT before the alpha transform
   unsigned char *d_cov = nullptr;  // per l: covered by some non-empty scale
   double *d_Phi2 = nullptr;
   int *d_his = nullptr;       // per scale bl_hi

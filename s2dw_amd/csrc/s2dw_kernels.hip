@@ -2553,8 +2553,8 @@ __device__ __forceinline__ void alpha_c2r_body_m(const AlphaArgs &a, int npt, do
   alpha_c2r_body<LOGM, BL, true>(a, npt, lds, bid, nb);
 }
 
-// alpha r2c (synthesis) of packed real rows, for scales whose beta stage does
-// the gamma-DFT: sequence t = row pair pidx = p0 + t of one g.
+// alpha r2c (synthesis) of packed real rows, without the gamma-DFT: sequence
+// t = row pair pidx = p0 + t of one g.
 template <int LOGM, int BL, int NT = kTN>
 __device__ __forceinline__ void alpha_r2c_body(const AlphaArgs &a, int npt, double2 *lds, int bid, int nb) {
   constexpr int LOGTS = clog2(NT * kTE);  // log2 of the workgroup's slots
@@ -2786,8 +2786,9 @@ __device__ __forceinline__ void alpha_syn_body(const AlphaArgs &a, int, double2 
     }
 }
 
-// gamma-DFT and quadrature weights (synthesis) as a pass of its own, for the
-// stages whose alpha or beta kernels are not on the workgroup engine; in place per (b, m):
+// gamma-DFT and quadrature weights (synthesis) as a pass of its own, for large
+// N (gamma_first) and for the stages whose beta kernels are not on the
+// workgroup engine; in place per (b, m):
 // U[ni][b][m] = wq[b] sum_g V[g][b][m] e^{-i n_ni pi g/N}; ni < nn <= N <= NMAX.
 template <int NMAX>
 __device__ __forceinline__ void gamma_syn_body(double2 *V, int hi, int N, int nn, const double *__restrict__ wq,
@@ -2815,10 +2816,23 @@ __device__ __forceinline__ void gamma_syn_body(double2 *V, int hi, int N, int nn
   }
 }
 
+// the scales of a launch: segment s owns workgroups [first[s], first[s+1])
+struct GammaSeg {
+  double2 *V;
+  const double *wq;
+  int hi;
+};
+struct GammaTab {
+  int nseg;
+  int first[kMaxSc + 1];
+  GammaSeg g[kMaxSc];
+};
 template <int NMAX>
-__global__ __launch_bounds__(256) void k_gamma_syn(double2 *V, int hi, int N, int nn, const double *__restrict__ wq,
-                                                   const double2 *__restrict__ eg) {
-  gamma_syn_body<NMAX>(V, hi, N, nn, wq, eg, (long long)blockIdx.x * blockDim.x + threadIdx.x);
+__global__ __launch_bounds__(256) void k_gamma_syn(const GammaTab t, int N, int nn, const double2 *__restrict__ eg) {
+  int s = 0;
+  for (int i = 1; i < t.nseg; ++i) s = (int)blockIdx.x >= t.first[i] ? i : s;
+  const GammaSeg &g = t.g[s];
+  gamma_syn_body<NMAX>(g.V, g.hi, N, nn, g.wq, eg, (long long)(blockIdx.x - t.first[s]) * blockDim.x + threadIdx.x);
 }
 
 // beta (synthesis) for one n-index: sequence t = 2*mc + r holds column
@@ -3034,6 +3048,30 @@ __global__ __launch_bounds__(NT, 3) void k_alpha_syn_o2(const AlphaArgs a0, cons
   }
 }
 
+// The same lengths without the gamma-DFT (gamma_first false): one packed row
+// pair of one g per workgroup, alpha_r2c_body's outputs.
+template <int R0, int R1, int R2, int NT = kOddNT, int SPLIT = kOddSplit>
+__global__ __launch_bounds__(NT, 3) void k_alpha_r2c_o2(const AlphaArgs a0, const AlphaArgs a1,
+                                                     const double2 *__restrict__ otw) {
+  constexpr int n = R0 * R1 * R2, hi = (n + 1) / 2;
+  __shared__ double2 lds[n];
+  const int half = gridDim.x >> 1, second = blockIdx.x >= (unsigned)half;
+  const AlphaArgs &a = second ? a1 : a0;
+  const int row = 2 * xcd_tile(blockIdx.x - (second ? half : 0), half);  // 2 hi g + 2 pidx
+  const double *w0 = a.W + (long long)row * n;
+  for (int k = threadIdx.x; k < n; k += NT) lds[k] = make_double2(w0[k], w0[n + k]);
+  lds_barrier();
+  odd_fft<R0, R1, R2, -1, NT, 1, SPLIT>(lds, otw);
+  const double h = 0.5 * a.scale;
+  double2 *v0 = a.V + (long long)row * hi;
+  for (int kk = threadIdx.x; kk < hi; kk += NT) {
+    const double2 zp = lds[kk];
+    const double2 zm = lds[kk ? n - kk : 0];
+    v0[kk] = make_double2(h * (zp.x + zm.x), h * (zp.y - zm.y));
+    v0[hi + kk] = make_double2(h * (zp.y + zm.y), -h * (zp.x - zm.x));
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Alpha stages and one-FFT-per-column beta stages on the three-stage engine
 // (Bluestein, M = 2^LOGM, M/16 threads, one sequence or column per
@@ -3153,6 +3191,44 @@ __global__ __launch_bounds__((1 << LOGM) / 16, 3) void k_alpha_syn16(const Alpha
   for (int r = 0; r < 8; ++r) {
     const int kk = threadIdx.x + NT * r;
     if (kk < hi) syn_store(a, us, kk, v[r], us.packed && kk ? dyn_lds[n - kk - hi] : v[r]);
+  }
+}
+
+// ... without the gamma-DFT: one packed row pair of one g per workgroup
+template <int LOGM>
+__global__ __launch_bounds__((1 << LOGM) / 16, 3) void k_alpha_r2c16(const AlphaArgs a0, const AlphaArgs a1, int half) {
+  constexpr int NT = (1 << LOGM) / 16;
+  extern __shared__ double2 dyn_lds[];
+  const bool second = (int)blockIdx.x >= half;
+  const AlphaArgs &a = second ? a1 : a0;
+  const int hi = a.hi, n = 2 * hi - 1;
+  const int row = 2 * xcd_tile(blockIdx.x - (second ? half : 0), half);  // 2 hi g + 2 pidx
+  const double *w0 = a.W + (long long)row * n;
+  double2 v[16];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const int k = threadIdx.x + NT * r, kk = k < n ? k : 0;
+    v[r] = cmulw<-1>(make_double2(w0[kk], w0[n + kk]), a.f.chirp[k]);  // chirp: zero for n <= k < M
+  }
+  team16_bluestein<LOGM, -1>(a.f, (double *)dyn_lds, v);
+#pragma unroll
+  for (int r = 0; r < 8; ++r) v[r] = cmulw<-1>(v[r], a.f.chirp[threadIdx.x + NT * r]);
+  lds_barrier();
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {  // Z(n - k), n - k >= hi, from the thread that holds it
+    const int k = threadIdx.x + NT * r;
+    if (k >= hi && k < n) dyn_lds[k - hi] = v[r];
+  }
+  lds_barrier();
+  const double h = 0.5 * a.scale;
+  double2 *v0 = a.V + (long long)row * hi;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const int kk = threadIdx.x + NT * r;
+    if (kk >= hi) continue;
+    const double2 zp = v[r], zm = kk ? dyn_lds[n - kk - hi] : v[r];
+    v0[kk] = make_double2(h * (zp.x + zm.x), h * (zp.y - zm.y));
+    v0[hi + kk] = make_double2(h * (zp.y + zm.y), -h * (zp.x - zm.x));
   }
 }
 
@@ -3619,6 +3695,24 @@ __global__ __launch_bounds__(kTN, 3) void k_alpha_syn_g(const SegTab t, const Al
   }
 }
 
+__global__ __launch_bounds__(kTN, 3) void k_alpha_r2c_g(const SegTab t, const AlphaArgs *__restrict__ args,
+                                                         const double *wbase) {
+  __shared__ double2 lds[lpad_size(kTS)];
+  const int s = seg_of(t, blockIdx.x), bid = blockIdx.x - t.first[s], nb = t.first[s + 1] - t.first[s];
+  AlphaArgs a = args[s];
+  a.W = const_cast<double *>(wbase) + a.woff;
+  switch (t.sel[s]) {
+    S2DW_SEL(alpha_r2c_body, 5, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_r2c_body, 6, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_r2c_body, 7, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_r2c_body, 8, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_r2c_body, 9, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_r2c_body, 10, 1, a, t.par[s], lds, bid, nb)
+    S2DW_SEL(alpha_r2c_body, 11, 1, a, t.par[s], lds, bid, nb)
+    default: alpha_r2c_body<0, -1>(a, t.par[s], lds, bid, nb); break;
+  }
+}
+
 __global__ __launch_bounds__(kTN, 3) void k_beta_syn_g(const SegTab t, const BetaSynArgs *__restrict__ args) {
   __shared__ double2 lds[lpad_size(kTS)];
   __shared__ double2 csum[kTN];
@@ -4022,13 +4116,53 @@ void launch_beta_syn(const TeamShape &t, const BetaSynArgs &y0, const BetaSynArg
   }
 }
 #undef S2DW_H2_CASES
-// packed real rows without the gamma-DFT, for the scales whose beta stage
-// does it (gamma_first)
-void launch_alpha_r2c(const TeamShape &t, const AlphaArgs &a, int npt, int blocks, hipStream_t st) {
+// packed real rows without the gamma-DFT
+void launch_alpha_r2c(const TeamShape &t, const AlphaArgs &a0, const AlphaArgs &a1, int npt, int half, int blocks,
+                      hipStream_t st) {
   const dim3 g(blocks);
-  if (t.bl && t.lg == 12) hipLaunchKernelGGL((k_alpha_r2c_t2<12, 1>), g, dim3(nt_of(12)), lds_of(12), st, a, a, npt, blocks);
-  else if (t.bl && t.lg == 13) hipLaunchKernelGGL((k_alpha_r2c_t2<13, 1>), g, dim3(nt_of(13)), lds_of(13), st, a, a, npt, blocks);
-  else hipLaunchKernelGGL((k_alpha_r2c_t2<0, -1>), g, dim3(kTN), 0, st, a, a, npt, blocks);
+  switch (t.bl ? t.lg : 0) {
+#define S2DW_X(LM)                                                                                        \
+  case LM:                                                                                                \
+    hipLaunchKernelGGL((k_alpha_r2c_t2<LM, 1>), g, dim3(nt_of(LM)), lds_of(LM), st, a0, a1, npt, half);   \
+    break;
+    S2DW_X(5) S2DW_X(6) S2DW_X(7) S2DW_X(8) S2DW_X(9) S2DW_X(10) S2DW_X(13)
+#undef S2DW_X
+    case 11: hipLaunchKernelGGL((k_alpha_r2c16<11>), g, dim3(128), lds16_of(11), st, a0, a1, half); break;
+    case 12: hipLaunchKernelGGL((k_alpha_r2c16<12>), g, dim3(256), lds16_of(12), st, a0, a1, half); break;
+    default: hipLaunchKernelGGL((k_alpha_r2c_t2<0, -1>), g, dim3(kTN), 0, st, a0, a1, npt, half); break;
+  }
+}
+
+void add_gamma(const Plan *p, GammaTab &t, int j) {
+  const Scale &s = p->sc[j];
+  t.first[t.nseg + 1] = t.first[t.nseg] + (int)((2LL * s.hi * s.hi + 255) / 256);
+  t.g[t.nseg++] = GammaSeg{p->d_tb + s.tb_off, p->d_wq + p->wq_off[j], s.hi};
+}
+void launch_gamma_syn(const Plan *p, const GammaTab &t, hipStream_t st) {
+  const int N = p->N, nn = (int)p->nlist.size();
+  const dim3 g(t.first[t.nseg]);
+  if (N <= 8) hipLaunchKernelGGL(k_gamma_syn<8>, g, dim3(256), 0, st, t, N, nn, p->eg);
+  else if (N <= 16) hipLaunchKernelGGL(k_gamma_syn<16>, g, dim3(256), 0, st, t, N, nn, p->eg);
+  else hipLaunchKernelGGL(k_gamma_syn<32>, g, dim3(256), 0, st, t, N, nn, p->eg);
+}
+
+// Whether the synthesis of a scale takes the gamma-DFT before the alpha
+// transform (alpha_syn_body) where both its FFT stages are on the workgroup
+// engine; a grouped launch takes the form of its largest scale.  The gather
+// reads every wavelet row once per n, N^2/2 reads per row pair, the pass on
+// its own moves N planes of f64 pairs twice.  FFT stages of a synthesis, us, before /
+// on its own: L = 128, N = 32 99 / 115; L = 256, N = 12 101 / 105, 16 133 / 130,
+// 32 347 / 310; L = 300, N = 12 189 / 187, 16 275 / 254, 32 717 / 582; L = 700,
+// N = 16 1296 / 1186; L = 512, N = 16 386 / 394, 20 522 / 518, 32 1043 / 909;
+// L = 1024, N = 16 1821 / 1849.  Scales of hi = 150 are even at N = 32.
+// Between 1.8 and 2.4 million N hi^2 the N planes of the pass on its own (60 to
+// 77 MB a scale) push the contraction's input out of the last-level cache and
+// the N/2 of the other do not: whole synthesis, us, L = 240, N = 32 1914 /
+// 2220, L = 256, N = 28 1837 / 2132; beyond, L = 300, N = 28 2687 / 2535.
+bool gamma_first(const Plan *p, int hi) {
+  const bool pow2 = hi > 256 && (hi & (hi - 1)) == 0;
+  const double planes = (double)p->N * hi * hi;
+  return hi < 200 || p->N < (pow2 ? 20 : 16) || (planes > 1.82e6 && planes < 2.4e6);
 }
 
 }  // namespace
@@ -4673,13 +4807,8 @@ int plan_build(Plan *p, int B, int N, int J, double alpha, const double *K, cons
     if (int e = upload(d_eg, eg.data(), eg.size() * sizeof(double2), p->stream)) return e;
     p->eg = d_eg;
     p->nlist = nlist;
-    // the synthesis takes the gamma-DFT before the alpha transform wherever
-    // both its FFT stages are on the workgroup engine: the n of one parity
-    // (N + n odd) give at most the N sequences per row pair that the packed
-    // real rows take (see alpha_syn_body)
     const auto z0 = std::find(nlist.begin(), nlist.end(), 0);
     p->z0 = z0 == nlist.end() ? -1 : (int)(z0 - nlist.begin());
-    p->gamma_first = !nlist.empty() && N <= kMaxCol;
   }
   // LDS: the generic FFT kernels need two buffers of the work length, the
   // wave-engine kernels one 64*E region per wave.
@@ -4709,7 +4838,7 @@ int plan_build(Plan *p, int B, int N, int J, double alpha, const double *K, cons
         {(const void *)k_alpha_c2r16<12, false>, lds16_of(12)}, {(const void *)k_alpha_c2r_t2<13, 1>, lds_of(13)},
         {(const void *)k_alpha_c2r16<12, true>, lds16_of(12)},  {(const void *)k_alpha_c2r_t2m<13, 1>, lds_of(13)},
         {(const void *)k_alpha_syn16<12>, lds16_of(12)},        {(const void *)k_alpha_syn_t2<13, 1>, lds_of(13)},
-        {(const void *)k_alpha_r2c_t2<12, 1>, lds_of(12)}, {(const void *)k_alpha_r2c_t2<13, 1>, lds_of(13)}};
+        {(const void *)k_alpha_r2c16<12>, lds16_of(12)},        {(const void *)k_alpha_r2c_t2<13, 1>, lds_of(13)}};
     for (const auto &b : big)
       if (b.lds + kCsumLds <= maxlds)
         S2DW_HIP_CHECK(hipFuncSetAttribute(b.fn, hipFuncAttributeMaxDynamicSharedMemorySize, b.lds));
@@ -4905,6 +5034,8 @@ int beta_sel(const TeamShape &t) { return t.h2 ? kSelH2 + 2 * t.lg + t.bl : 0; }
 // tables go in the kernel arguments, the stage arguments in device tables.
 struct Group {
   bool ana = false, syn = false;
+  bool first = true;  // synthesis: gamma-DFT before the alpha transform
+  GammaTab gm{};      // else its pass
   SegTab ba{}, ac{}, am{}, ar{}, bs{};  // am: alpha c2r reducing to moments
   BetaAnaArgs *d_ba = nullptr;
   AlphaArgs *d_ac = nullptr, *d_ar = nullptr;
@@ -4914,7 +5045,8 @@ struct Group {
 struct GroupState {
   Group g[2];                        // 1: scales 2..J, or 0..J on one stream (0 unused)
   std::vector<char> in_ana, in_syn;  // per scale: runs in a group
-  bool pair = false;                 // scales 0 and 1 run as pair launches
+  bool pair = false;                 // scales 0 and 1 run as pair launches in the analysis
+  bool pair_syn = false;             // ... and in the synthesis
 };
 
 void free_groups(Plan *p) {
@@ -4933,14 +5065,16 @@ int build_group(Plan *p, GroupState *gs, int gi, int j0, int j1) {
   std::vector<BetaSynArgs> bs;
   std::vector<int> taken;
   bool ok = j1 - j0 >= 2 || (gi == 1 && j1 > j0);
-  const bool syn_ok = p->gamma_first;
   // workgroups that the three-stage engine would take of the analysis alpha launch
   auto wg16_of = [&](const Scale &s, const TeamShape &t) { return (s.hi + (4096 >> t.lg) - 1) / (4096 >> t.lg) * N; };
-  int wg16 = 0;
+  int wg16 = 0, hmax = 0;
   for (int j = j0; j < j1; ++j) {
     const TeamShape t = scale_empty(p->sc[j]) ? TeamShape{} : alpha_shape(p, p->ffts[p->sc[j].fa]);
     if (t.bl && (t.lg == 10 || t.lg == 11)) wg16 += wg16_of(p->sc[j], t);
+    if (t.lg >= 0 && t.lg <= kLogTS) hmax = std::max(hmax, p->sc[j].hi);
   }
+  const bool syn_ok = !p->nlist.empty() && N <= kMaxCol;
+  G.first = gamma_first(p, hmax);
   for (int j = j0; j < j1 && ok; ++j) {
     const Scale &s = p->sc[j];
     if (scale_empty(s)) {
@@ -4966,7 +5100,6 @@ int build_group(Plan *p, GroupState *gs, int gi, int j0, int j1) {
       t.par[i] = par;
     };
     add(G.ba, nmt * N, beta_sel(tb), nmt);
-    add(G.bs, nmt * nn, beta_sel(tb), nmt);
     // analysis, work length 2048, and 1024 where the launch has a workgroup per
     // CU of these: the three-stage engine; it holds twice the sequences per
     // workgroup.  This launch, on it and on the radix-8 body, us: L = 256, N = 2
@@ -4979,11 +5112,14 @@ int build_group(Plan *p, GroupState *gs, int gi, int j0, int j1) {
     if (e16) add(G.ac, np16 * N, kSel16 + ta.lg, np16);
     else add(G.ac, npt * N, alpha_sel(ta), npt);
     add(G.am, npt * N, alpha_sel(ta), npt);
-    add(G.ar, syn_blocks(p, s.hi, ta.per), alpha_sel(ta), 0);
     taken.push_back(j);
     ba.push_back(b);
     a.moff = 8 * p->momf_rec0[j];
     ac.push_back(a);
+    if (G.first) add(G.ar, syn_blocks(p, s.hi, ta.per), alpha_sel(ta), 0);
+    else add(G.ar, npt * N, alpha_sel(ta), npt);
+    add_gamma(p, G.gm, j);
+    add(G.bs, nmt * nn, beta_sel(tb), nmt);
     ar.push_back(r);
     bs.push_back(y);
   }
@@ -5052,10 +5188,12 @@ int build_groups(Plan *p) {
     if (int e = build_group(p, gs, 1, 2, Jp1)) return e;
   // scales 0 and 1 as one pair launch per stage when they have the same
   // FFT specs and run on the workgroup engine
-  if (!all_in && Jp1 >= 2 && !scale_empty(p->sc[0]) && !scale_empty(p->sc[1]) && p->sc[0].fa == p->sc[1].fa &&
+  if (Jp1 >= 2 && !scale_empty(p->sc[0]) && !scale_empty(p->sc[1]) && p->sc[0].fa == p->sc[1].fa &&
       p->sc[0].fb == p->sc[1].fb && p->sc[0].hi == p->sc[1].hi &&
-      beta_shape(p, p->ffts[p->sc[0].fb], p->sc[0].hi).lg >= 0 && alpha_shape(p, p->ffts[p->sc[0].fa]).lg >= 0)
-    gs->pair = true;
+      beta_shape(p, p->ffts[p->sc[0].fb], p->sc[0].hi).lg >= 0 && alpha_shape(p, p->ffts[p->sc[0].fa]).lg >= 0) {
+    gs->pair = !gs->in_ana[0];
+    gs->pair_syn = !gs->in_syn[0] && !p->nlist.empty() && N <= kMaxCol;
+  }
   for (int j = 0; j < Jp1; ++j)
     if (!scale_empty(p->sc[j]) && !gs->in_ana[j] && !(gs->pair && j < 2)) mok = false;
   p->momf_ok = mok;
@@ -5387,14 +5525,22 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
   }
   const GroupState *grp = static_cast<const GroupState *>(p->groups);
   const int nn_all = (int)p->nlist.size();
-  const bool pair = grp && grp->pair && p->gamma_first;
+  const bool pair = grp && grp->pair_syn;
   for (int gi = 1; gi >= 0; --gi) {
     if (!grp || !grp->g[gi].syn) continue;
     const Group &G = grp->g[gi];
     hipStream_t sg = (conc && gi == 1) ? p->aux : st;
     {
       StageTimer tm(p, 10);
-      hipLaunchKernelGGL(k_alpha_syn_g, dim3(G.ar.first[G.ar.nseg]), dim3(kTN), 0, sg, G.ar, G.d_ar, d_wav);
+      if (G.first)
+        hipLaunchKernelGGL(k_alpha_syn_g, dim3(G.ar.first[G.ar.nseg]), dim3(kTN), 0, sg, G.ar, G.d_ar, d_wav);
+      else
+        hipLaunchKernelGGL(k_alpha_r2c_g, dim3(G.ar.first[G.ar.nseg]), dim3(kTN), 0, sg, G.ar, G.d_ar, d_wav);
+      S2DW_HIP_CHECK(hipGetLastError());
+    }
+    if (!G.first) {
+      StageTimer tm(p, 10);
+      launch_gamma_syn(p, G.gm, sg);
       S2DW_HIP_CHECK(hipGetLastError());
     }
     StageTimer tm(p, 10);
@@ -5402,6 +5548,7 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
     S2DW_HIP_CHECK(hipGetLastError());
   }
   if (pair) {
+    const bool first = gamma_first(p, p->sc[0].hi);
     AlphaArgs a0 = make_alpha(p, 0, true), a1 = make_alpha(p, 1, true);
     const TeamShape ta = alpha_shape(p, a0.f);
     a0.logT = a1.logT = team_logTw(p, a0.f, false);
@@ -5409,14 +5556,24 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
     a1.W = const_cast<double *>(d_wav + p->sc[1].wav_off);
     {
       StageTimer tm(p, 5);
-      const int nb = syn_blocks(p, a0.hi, p->d_otw ? 1 : ta.per);
-      if (p->d_otw)
+      const int nb = syn_blocks(p, a0.hi, p->d_otw ? 1 : ta.per), npt = (a0.hi + ta.per - 1) / ta.per;
+      if (first && p->d_otw)
         hipLaunchKernelGGL((k_alpha_syn_o2<31, 11, 3>), dim3(2 * nb), dim3(kOddNT), 0, st, a0, a1, p->d_otw);
-      else
+      else if (first)
         launch_alpha_syn(ta, a0, a1, 0, nb, 2 * nb, st);
+      else if (p->d_otw)
+        hipLaunchKernelGGL((k_alpha_r2c_o2<31, 11, 3>), dim3(2 * a0.hi * N), dim3(kOddNT), 0, st, a0, a1, p->d_otw);
+      else
+        launch_alpha_r2c(ta, a0, a1, npt, npt * N, 2 * npt * N, st);
       S2DW_HIP_CHECK(hipGetLastError());
     }
     StageTimer tm(p, 6);
+    if (!first) {
+      GammaTab gt{};
+      for (int j : {0, 1}) add_gamma(p, gt, j);
+      launch_gamma_syn(p, gt, st);
+      S2DW_HIP_CHECK(hipGetLastError());
+    }
     BetaSynArgs y0 = make_beta_syn(p, 0), y1 = make_beta_syn(p, 1);
     const TeamShape tb = beta_shape(p, y0.f, y0.hi);
     y0.logT = y1.logT = team_logTw(p, y0.f, true);
@@ -5442,10 +5599,10 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
       const TeamShape ts = alpha_shape(p, al.f);
       if (ts.lg >= 0) {
         al.logT = team_logTw(p, al.f, false);
-        gamma_done = team_beta && p->gamma_first;
+        gamma_done = team_beta && gamma_first(p, s.hi);
         const int npt = (s.hi + ts.per - 1) / ts.per, nb = syn_blocks(p, s.hi, ts.per);
         if (gamma_done) launch_alpha_syn(ts, al, al, 0, nb, nb, sj);
-        else launch_alpha_r2c(ts, al, npt, npt * N, sj);
+        else launch_alpha_r2c(ts, al, al, npt, npt * N, npt * N, sj);
       } else if (ws.ok) {
         al.logT = ws.logTw;
         const int per = ws.WPB << ws.logTw;
@@ -5466,11 +5623,9 @@ int run_synthesis(Plan *p, double2 *d_flm, const double *d_wav, const double2 *d
       const WaveShape ws = wave_shape(p, b.f);
       if (team_beta) {
         if (!gamma_done) {
-          const dim3 gg((unsigned)((2LL * s.hi * s.hi + 255) / 256));
-          double2 *Vj = p->d_tb + s.tb_off;
-          if (N <= 8) hipLaunchKernelGGL(k_gamma_syn<8>, gg, dim3(256), 0, sj, Vj, s.hi, N, nn, b.wq, b.eg);
-          else if (N <= 16) hipLaunchKernelGGL(k_gamma_syn<16>, gg, dim3(256), 0, sj, Vj, s.hi, N, nn, b.wq, b.eg);
-          else hipLaunchKernelGGL(k_gamma_syn<32>, gg, dim3(256), 0, sj, Vj, s.hi, N, nn, b.wq, b.eg);
+          GammaTab gt{};
+          add_gamma(p, gt, j);
+          launch_gamma_syn(p, gt, sj);
           S2DW_HIP_CHECK(hipGetLastError());
         }
         b.logT = team_logTw(p, b.f, true);
