@@ -2279,12 +2279,11 @@ __device__ __forceinline__ double2 chirp_in(const FftSpec &f, double2 x, int k) 
 
 // beta (analysis): sequence t = 2*mc + r holds column m = m0 + mc and output
 // parity r; the workgroup reads each Tg element once for both parities.
-template <int LOGM, int BL>
 __device__ __forceinline__ void beta_ana_body(const BetaAnaArgs &a, int nmt, double2 *lds, int bid, int nb) {
   const FftSpec &f = a.f;
-  const bool bluestein = BL >= 0 ? BL != 0 : f.bluestein != 0;
-  const int hi = a.hi, n = 2 * hi, e8 = 8 * hi, M = LOGM > 0 ? 1 << LOGM : f.M;
-  const int logTw = LOGM > 0 ? kLogTS - LOGM : a.logT, Tw = 1 << logTw, logMC = logTw - 1, MC = Tw >> 1;
+  const bool bluestein = f.bluestein != 0;
+  const int hi = a.hi, n = 2 * hi, e8 = 8 * hi, M = f.M;
+  const int logTw = a.logT, Tw = 1 << logTw, logMC = logTw - 1, MC = Tw >> 1;
   const int tile = xcd_tile(bid, nb);
   const int g = tile / nmt, m0 = (tile - g * nmt) * MC;
   {
@@ -2334,7 +2333,6 @@ __device__ __forceinline__ void beta_ana_body(const BetaAnaArgs &a, int nmt, dou
       a.Tb[(long long)g * n * hi + (2 * bp + r) * a.tbb + m * a.tbm] = y;
     }
   }
-  (void)M;
 }
 
 // Rows p = rb, q = rb + sb of a packed pair at the lane's own k: lanes 2i and
@@ -2722,8 +2720,8 @@ __device__ __forceinline__ void syn_store(const AlphaArgs &a, const SynSeq &sq, 
 
 // A thread works on one sequence: M/8 consecutive threads per sequence.  The
 // length 2hi - 1 is odd, so this is always Bluestein, n <= M/2, M >= 8.
-template <int LOGM, int, int NT = kTN>
-__device__ __forceinline__ void alpha_syn_body(const AlphaArgs &a, int, double2 *lds, int bid, int nb) {
+template <int LOGM, int NT = kTN>
+__device__ __forceinline__ void alpha_syn_body(const AlphaArgs &a, double2 *lds, int bid, int nb) {
   constexpr int LOGTS = clog2(NT * kTE);
   const FftSpec &f = a.f;
   const int hi = a.hi, n = 2 * hi - 1, logM = LOGM > 0 ? LOGM : ilog2(f.M), M = 1 << logM;
@@ -2837,13 +2835,12 @@ __global__ __launch_bounds__(256) void k_gamma_syn(const GammaTab t, int N, int 
 
 // beta (synthesis) for one n-index: sequence t = 2*mc + r holds column
 // m = m0 + mc and m' parity r; input U from k_gamma_syn.
-template <int LOGM, int BL>
 __device__ __forceinline__ void beta_syn_body(const BetaSynArgs &a, const double2 *V, double2 *Vt, const double2 *tw8,
                                               int nmt, double2 *lds, int bid, int nb) {
   const FftSpec &f = a.f;
-  const bool bluestein = BL >= 0 ? BL != 0 : f.bluestein != 0;
-  const int hi = a.hi, n2 = 2 * hi, e8 = 8 * hi, M = LOGM > 0 ? 1 << LOGM : f.M;
-  const int logTw = LOGM > 0 ? kLogTS - LOGM : a.logT, Tw = 1 << logTw, logMC = logTw - 1, MC = Tw >> 1;
+  const bool bluestein = f.bluestein != 0;
+  const int hi = a.hi, n2 = 2 * hi, M = f.M;
+  const int logTw = a.logT, Tw = 1 << logTw, logMC = logTw - 1, MC = Tw >> 1;
   const int tile = xcd_tile(bid, nb);
   const int ni = tile / nmt, m0 = (tile - ni * nmt) * MC;
   const double2 *U = V + (long long)ni * n2 * hi;
@@ -2927,11 +2924,10 @@ inline bool big_fft(const FftSpec &f) { return f.bluestein && f.M > kTS && f.M <
   __shared__ double2 fix_lds[(LOGM) > kLogTS ? 1 : lpad_size(kTS)]; \
   double2 *lds = (LOGM) > kLogTS ? dyn_lds : fix_lds;
 
-template <int LOGM, int BL>
 __global__ __launch_bounds__(kTN, 3) void k_beta_ana_t2(const BetaAnaArgs a0, const BetaAnaArgs a1, int nmt, int half) {
   __shared__ double2 lds[lpad_size(kTS)];
   const bool second = (int)blockIdx.x >= half;
-  beta_ana_body<LOGM, BL>(second ? a1 : a0, nmt, lds, blockIdx.x - (second ? half : 0), half);
+  beta_ana_body(second ? a1 : a0, nmt, lds, blockIdx.x - (second ? half : 0), half);
 }
 template <int LOGM, int BL>
 __global__ __launch_bounds__(nt_of(LOGM), occ_of(LOGM)) void k_alpha_c2r_t2(const AlphaArgs a0, const AlphaArgs a1,
@@ -2960,7 +2956,7 @@ __global__ __launch_bounds__(nt_of(LOGM), occ_of(LOGM)) void k_alpha_syn_t2(cons
                                                                            int npt, int half) {
   S2DW_SLOTS(LOGM)
   const bool second = (int)blockIdx.x >= half;
-  alpha_syn_body<LOGM, BL, nt_of(LOGM)>(second ? a1 : a0, npt, lds, blockIdx.x - (second ? half : 0), half);
+  alpha_syn_body<LOGM, nt_of(LOGM)>(second ? a1 : a0, lds, blockIdx.x - (second ? half : 0), half);
 }
 
 // Alpha stages of the full-band pair on the odd-length engine, length
@@ -3232,12 +3228,11 @@ __global__ __launch_bounds__((1 << LOGM) / 16, 3) void k_alpha_r2c16(const Alpha
   }
 }
 
-template <int LOGM, int BL>
 __global__ __launch_bounds__(kTN, 3) void k_beta_syn_t2(const BetaSynArgs a, const double2 *V1, double2 *Vt1,
                                                         const double2 *tw81, int nmt, int half) {
   __shared__ double2 lds[lpad_size(kTS)];
   const bool second = (int)blockIdx.x >= half;
-  beta_syn_body<LOGM, BL>(a, second ? V1 : a.V, second ? Vt1 : a.Vt, second ? tw81 : a.tw8, nmt, lds,
+  beta_syn_body(a, second ? V1 : a.V, second ? Vt1 : a.Vt, second ? tw81 : a.tw8, nmt, lds,
                           blockIdx.x - (second ? half : 0), half);
 }
 
@@ -3636,7 +3631,7 @@ __global__ __launch_bounds__(kTN, 3) void k_beta_ana_g(const SegTab t, const Bet
   const BetaAnaArgs a = args[s];
   switch (t.sel[s]) {
     S2DW_SEL_H2_ALL(beta_ana_h2_body, a, t.par[s], lds, bid, nb)
-    default: beta_ana_body<0, -1>(a, t.par[s], lds, bid, nb); break;
+    default: beta_ana_body(a, t.par[s], lds, bid, nb); break;
   }
 }
 
@@ -3684,14 +3679,11 @@ __global__ __launch_bounds__(kTN, 3) void k_alpha_syn_g(const SegTab t, const Al
   AlphaArgs a = args[s];
   a.W = const_cast<double *>(wbase) + a.woff;
   switch (t.sel[s]) {
-    S2DW_SEL(alpha_syn_body, 5, 1, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(alpha_syn_body, 6, 1, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(alpha_syn_body, 7, 1, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(alpha_syn_body, 8, 1, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(alpha_syn_body, 9, 1, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(alpha_syn_body, 10, 1, a, t.par[s], lds, bid, nb)
-    S2DW_SEL(alpha_syn_body, 11, 1, a, t.par[s], lds, bid, nb)
-    default: alpha_syn_body<0, -1>(a, t.par[s], lds, bid, nb); break;
+#define S2DW_X(LM) \
+  case 2 * (LM) + 1: alpha_syn_body<LM>(a, lds, bid, nb); break;
+    S2DW_X(5) S2DW_X(6) S2DW_X(7) S2DW_X(8) S2DW_X(9) S2DW_X(10) S2DW_X(11)
+#undef S2DW_X
+    default: alpha_syn_body<0>(a, lds, bid, nb); break;
   }
 }
 
@@ -3720,7 +3712,7 @@ __global__ __launch_bounds__(kTN, 3) void k_beta_syn_g(const SegTab t, const Bet
   const BetaSynArgs &a = args[s];
   switch (t.sel[s]) {
     S2DW_SEL_H2_ALL(beta_syn_h2_body, a, a.V, a.Vt, a.tw8, t.par[s], lds, csum, bid, nb)
-    default: beta_syn_body<0, -1>(a, a.V, a.Vt, a.tw8, t.par[s], lds, bid, nb); break;
+    default: beta_syn_body(a, a.V, a.Vt, a.tw8, t.par[s], lds, bid, nb); break;
   }
 }
 #undef S2DW_SEL
@@ -4092,7 +4084,7 @@ void launch_beta_ana(const TeamShape &t, const BetaAnaArgs &b0, const BetaAnaArg
     case 2 * 12 + 1:
       hipLaunchKernelGGL((k_beta_ana16<12>), g, dim3(256), lds16_of(12), st, b0, b1, nmt, half);
       break;
-    default: hipLaunchKernelGGL((k_beta_ana_t2<0, -1>), g, dim3(kTN), 0, st, b0, b1, nmt, half); break;
+    default: hipLaunchKernelGGL(k_beta_ana_t2, g, dim3(kTN), 0, st, b0, b1, nmt, half); break;
   }
 }
 void launch_beta_syn(const TeamShape &t, const BetaSynArgs &y0, const BetaSynArgs &y1, int nmt, int half, int blocks,
@@ -4112,7 +4104,7 @@ void launch_beta_syn(const TeamShape &t, const BetaSynArgs &y0, const BetaSynArg
     case 2 * 12 + 1:
       hipLaunchKernelGGL((k_beta_syn16<12>), g, dim3(256), lds16_of(12), st, y0, y1.V, y1.Vt, y1.tw8, nmt, half);
       break;
-    default: hipLaunchKernelGGL((k_beta_syn_t2<0, -1>), g, dim3(kTN), 0, st, y0, y1.V, y1.Vt, y1.tw8, nmt, half); break;
+    default: hipLaunchKernelGGL(k_beta_syn_t2, g, dim3(kTN), 0, st, y0, y1.V, y1.Vt, y1.tw8, nmt, half); break;
   }
 }
 #undef S2DW_H2_CASES
