@@ -25,6 +25,7 @@ from __future__ import annotations
 import argparse
 import json
 import os
+import re
 import statistics
 import sys
 import time
@@ -52,19 +53,35 @@ def seeded_flm(B, seed, red=True):
     return f
 
 
-def contraction_cmacs(hi, lo, N):
-    """Useful complex MACs of the l-contraction, per transform:
-    analysis sum_j sum_{l=lo_j+1}^{hi_j-1} n_a(l) (l+1)^2 with n_a(l) = #{n: |n| <= min(N-1,l), N+n odd};
-    synthesis the same with n >= 0 only."""
-    ana = syn = 0
+def contraction_flops(hi, lo, N):
+    """Real flops of the l-contraction, per transform: 4 (one real by complex
+    multiply-add) per column n, m' and m of every l of every scale, without the
+    recursions of the Wigner values.  Returns (both signs of n, n >= 0 only):
+    the second is what the synthesis and the analysis by parity of l do, where
+    the columns n and -n share their sums; the other analysis kernels do the
+    first."""
+    both = pos = 0
     for h, lo_ in zip(hi, lo):
         for l in range(lo_ + 1, h):
             nmax = min(N - 1, l)
-            na = sum(1 for n in range(-nmax, nmax + 1) if (N + n) % 2)
-            ns = sum(1 for n in range(0, nmax + 1) if (N + n) % 2)
-            ana += na * (l + 1) ** 2
-            syn += ns * (l + 1) ** 2
-    return ana, syn
+            both += sum(1 for n in range(-nmax, nmax + 1) if (N + n) % 2) * (l + 1) ** 2
+            pos += sum(1 for n in range(0, nmax + 1) if (N + n) % 2) * (l + 1) ** 2
+    return 4.0 * both, 4.0 * pos
+
+
+def analysis_contraction(precision, tuned):
+    """(kernel, the unit that bounds it, both signs of n) of the analysis
+    contraction that a plan runs, from the autotuner's report of the times."""
+    if precision != "fp64":
+        return "k_ana_contract_split", "mfma", True
+    # the analysis candidates come before the report's first semicolon
+    times = re.findall(r"(parity|mfma-wave|mfma-staged|valu-p\d) ([0-9.]+) ms", tuned.split(";")[0])
+    best = min(times, key=lambda t: float(t[1]))[0] if times else "parity"
+    if best == "parity":
+        return "k_ana_contract_par", "valu-fp64", False
+    if best.startswith("mfma"):
+        return "k_ana_contract_mfma", "mfma", True
+    return "k_ana_contract<", "valu-fp64", True
 
 
 def stage_bytes(hi, lo, N, ncs, grouped=True):
@@ -335,24 +352,26 @@ def bench_serve(args, precision=0):
     return out
 
 
-# stage name -> kernel whose launches dominate it
-STAGE_KERNEL = {"ana_contract": "k_ana_contract_par", "syn_contract": "k_syn_contract_mfma",
+# stage name -> kernel whose launches dominate it (the analysis contraction's is
+# the one the plan runs)
+STAGE_KERNEL = {"syn_contract": "k_syn_contract_mfma",
                 "ana_beta_fft": "k_beta_ana_h2", "ana_alpha_c2r": "k_alpha_c2r_o2",
                 "syn_alpha_r2c": "k_alpha_syn_o2", "syn_beta_fft": "k_beta_syn_h2",
                 "ana_small_ffts": "k_alpha_c2r_g", "syn_small_ffts": "k_alpha_syn_g"}
 
 
-def load_traffic(stage):
+def load_traffic(kern):
+    """HBM bytes per dispatch of the instance of a kernel that moves the most, or
+    None where the counter run had no such kernel."""
     try:
         with open(TRAFFIC_JSON) as fh:
             data = json.load(fh)["kernels"]
     except (OSError, ValueError, KeyError):
         return None
-    kern = STAGE_KERNEL.get(stage)
-    hits = [v for k, v in data.items() if kern and k.startswith(kern)]
+    hits = [v for k, v in data.items() if k.startswith(kern)]
     if not hits:
         return None
-    return sum(h["hbm_bytes"] * h["dispatches"] for h in hits) / sum(h["dispatches"] for h in hits)
+    return max(hits, key=lambda h: h["hbm_bytes"] * h["dispatches"])["hbm_bytes"]
 
 
 def bench_pipelined(args, L, N, J, K, Phi2, S, prec, d_f, flm):
@@ -646,7 +665,10 @@ def main():
 
     hi, lo = plan.bl_hi, plan.bl_lo
     out_offs = list(plan.wav_offsets)
-    ana_cmac, syn_cmac = contraction_cmacs(hi, lo, N)
+    both, pos = contraction_flops(hi, lo, N)
+    ana_kernel, ana_bound, ana_both = analysis_contraction(args.precision, tuned)
+    contract = {"ana_contract": (ana_kernel, ana_bound, both if ana_both else pos),
+                "syn_contract": (STAGE_KERNEL["syn_contract"], "mfma", pos)}
     grouped = st.get("ana_small_ffts", (0.0, 0))[1] > 0
     sb = stage_bytes(hi, lo, N, ncs=sum(1 for n in range(N) if (N + n) % 2), grouped=grouped)
     stages = {}
@@ -658,27 +680,27 @@ def main():
     dom = max(stages, key=lambda k: stages[k]["ms_per_step"])
     nl = max(1.0, stages[dom]["launches_per_step"])
     launch_ms = stages[dom]["ms_per_step"] / nl
-    traffic = load_traffic(dom)
-    if dom in ("ana_contract", "syn_contract"):
-        cm = ana_cmac if dom == "ana_contract" else syn_cmac
-        work = 8.0 * cm / nl  # 8 real flops per useful complex MAC
+    kern = contract[dom][0] if dom in contract else STAGE_KERNEL.get(dom, dom)
+    traffic = load_traffic(kern)
+    if dom in contract:
+        work = contract[dom][2] / nl
         achieved = work / (launch_ms * 1e-3) / 1e12
-        roof = {"bound": "mfma", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
+        roof = {"bound": contract[dom][1], "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                 "frac": achieved / FP64_PEAK_TFLOPS, "traffic": traffic,
-                "kernel": STAGE_KERNEL.get(dom, dom), "stage": dom, "avg_launch_ms": launch_ms,
-                "work_per_launch": work, "work_unit": "flop (8 per useful complex MAC)"}
+                "kernel": kern, "stage": dom, "avg_launch_ms": launch_ms, "work_per_launch": work,
+                "work_unit": "flop (4 per real by complex multiply-add of a column, without the recursions)"}
     else:
         work = sb.get(dom, 0) / nl
         achieved = work / (launch_ms * 1e-3) / 1e9
         roof = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                "kernel": STAGE_KERNEL.get(dom, dom), "stage": dom, "avg_launch_ms": launch_ms,
+                "kernel": kern, "stage": dom, "avg_launch_ms": launch_ms,
                 "work_per_launch": work, "work_unit": "byte (compulsory)"}
     contraction = {}
-    for name, cm in (("ana_contract", ana_cmac), ("syn_contract", syn_cmac)):
+    for name, (kname, _, work) in contract.items():
         if name in stages:
-            tf = 8.0 * cm / (stages[name]["ms_per_step"] * 1e-3) / 1e12
-            contraction[name] = {"tflops": tf, "frac_fp64_peak": tf / FP64_PEAK_TFLOPS}
+            tf = work / (stages[name]["ms_per_step"] * 1e-3) / 1e12
+            contraction[name] = {"kernel": kname, "tflops": tf, "frac_fp64_peak": tf / FP64_PEAK_TFLOPS}
     ffts = {}
     for name, byts in sb.items():
         if name in stages:
