@@ -71,8 +71,8 @@ __device__ __forceinline__ double row_rec(double b, double x, double y) {
 //
 // Measured (N = 8, device time of the kernel; before: the FP64 MFMA kernel
 // with independent waves): L = 1024 1252 -> 447 us, 512 157 -> 98, 300 92 -> 59;
-// N = 4, L = 181 53 -> 28; N = 3, L = 64 35 -> 16.  At L = 1024 54% of the
-// cycles issue FP64; at L <= 512 the longest chains (m', m ~ 0: L steps) end
+// N = 4, L = 181 53 -> 28; N = 3, L = 64 35 -> 16.  At L = 1024 FP64 issues
+// in 69% of the cycles (FMAs 53%, products 16%); at L <= 512 the longest chains (m', m ~ 0: L steps) end
 // alone on their SIMDs and their latency bounds the kernel.
 constexpr int G = kParG, WV = kParWv;
 template <int NH>

@@ -768,10 +768,12 @@ __device__ __forceinline__ void team_fft_core(const FftSpec &s, double2 *buf, in
 // Three stages instead of the radix-8 engine's four, the first forward stage
 // from values the caller holds in registers, the last backward stage left in
 // registers, and the stages that meet at the filter joined in registers: the
-// slots are written four times and read four times per transform, where the
-// radix-8 engine of 512 threads writes and reads them eight times each and
+// slots are written and read in four exchanges per transform, each as two
+// half-width passes (real and imaginary parts, exchange16), where the radix-8
+// engine of 512 threads writes and reads whole values eight times each and
 // spills (its four stages of twiddles stay in registers: 128 of 128 VGPRs;
-// here 2 waves per SIMD leave 256).
+// here three waves per SIMD leave 168, and two 256 for the moments form of
+// M = 4096).
 // Physical slot of logical slot i: i + i/16.  Consecutive slots and slots 8 or
 // 16 apart, the patterns of the stages, fall in distinct banks over 16 lanes,
 // and every stage's slots are one base per thread plus compile-time offsets

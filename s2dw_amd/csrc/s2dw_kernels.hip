@@ -5022,8 +5022,8 @@ int beta_sel(const TeamShape &t) { return t.h2 ? kSelH2 + 2 * t.lg + t.bl : 0; }
 // Grouped launches (all on the workgroup FFT engine): the two full-band
 // scales j = 0, 1 (same shapes) in one launch per stage on the main stream,
 // and the small scales j >= 2 in one launch per stage on the helper stream:
-// analysis beta + alpha c2r, synthesis alpha (with the gamma-DFT) + beta.  Segment
-// tables go in the kernel arguments, the stage arguments in device tables.
+// analysis beta + alpha c2r, synthesis alpha (with the gamma-DFT, or its pass
+// after it) + beta.  Segment tables go in the kernel arguments, the stage arguments in device tables.
 struct Group {
   bool ana = false, syn = false;
   bool first = true;  // synthesis: gamma-DFT before the alpha transform
@@ -5046,9 +5046,10 @@ void free_groups(Plan *p) {
   p->groups = nullptr;
 }
 
-// Builds group gi from the scales [j0, j1); all must be non-empty and run
-// on the workgroup engine, else the group stays off (its scales launch one
-// by one).
+// Builds group gi from the scales [j0, j1).  Empty scales are left out (they
+// are filled one by one).  In a group of the scales from 2 on, so are scales
+// beyond the kTN-thread engine (they launch one by one); a group that starts
+// at scale 0 stays off if it has one.
 int build_group(Plan *p, GroupState *gs, int gi, int j0, int j1) {
   const int N = p->N, nn = (int)p->nlist.size();
   Group &G = gs->g[gi];
