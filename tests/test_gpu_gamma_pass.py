@@ -42,3 +42,29 @@ def test_gamma_pass(B, N, alpha, monkeypatch):
     torch.cuda.synchronize()
     assert torch.isfinite(out[0]).all() and torch.isfinite(out[1]).all()
     assert float((out[0] - out[1]).abs().max()) <= TOL
+
+
+@pytest.mark.parametrize("B,N", [(256, 16), (512, 20)])
+def test_gamma_pass_graph(B, N):
+    """Replays of the captured synthesis (one stream, two streams), with other
+    work between them, repeat the eager result bit for bit."""
+    import torch
+
+    print(f"gamma pass graph B={B} N={N}", flush=True)
+    J = min(4, core.s2dw_core_comp_Jmax(B, 2.0))
+    K, Phi2, _ = core.s2dw_core_init_kernels(J, B, 2.0)
+    S = core.s2dw_core_init_directionality(B, N)
+    p = core.Plan(B, N, J, 2.0, K, Phi2, S)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(B)
+    wav = torch.randn(p.empty_wav().shape, dtype=torch.float64, device="cuda", generator=g) / (2.0 * B)
+    sc = torch.zeros_like(p.empty_scoeff())
+    want, out = p.empty_flm(), p.empty_flm()
+    p.synthesis(wav, sc, want)
+    torch.cuda.synchronize()
+    p.set_graphs(True)
+    for _ in range(4):
+        out.zero_()
+        p.synthesis(wav, sc, out)
+        torch.cuda.synchronize()
+        assert torch.equal(torch.view_as_real(out), torch.view_as_real(want))
